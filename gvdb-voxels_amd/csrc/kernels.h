@@ -453,11 +453,17 @@ struct RenderArgs {
     Tree t;
     ScnBlock s;
     const float4* tf;
+    int tf_ramp;            // the table is tf_a + (i / TF_SIZE) tf_d
+    float tf_a[4], tf_d[4];
     const void* atlas;
     void* out;
     int out_float;
     int shading;
     int atlas_type;
+    // set by the launcher: ceil(2^32 / padded brick side), and 1 / the step and 1 / the value range where they are
+    // powers of two (0: divide)
+    uint32_t br_inv;
+    float step_inv, vr_inv;
     int tile_w;          // pixel tile of one 64-lane workgroup: tile_w x (64 / tile_w); set by the launcher
     const uint32_t* clr; // the colour channel (uchar4 per voxel, SetColorChannel), or null
 };

@@ -802,6 +802,15 @@ int Volume::linear_tf(float t0, float t1, const float a[4], const float b[4]) {
         float x = float(k - n0) / float(n1 - n0);
         for (int c = 0; c < 4; c++) tf_host[4 * k + c] = a[c] + x * (b[c] - a[c]);
     }
+    // one ramp over the whole table is remembered: the march evaluates it as
+    // this loop does, instead of reading the table
+    if (n1 > n0) {
+        tf_ramp_ = n0 == 0 && n1 == TF_SIZE;
+        for (int c = 0; c < 4; c++) {
+            tf_a_[c] = a[c];
+            tf_d_[c] = b[c] - a[c];
+        }
+    }
     tf_committed = false;
     return GVDB_OK;
 }

@@ -144,6 +144,8 @@ public:
     float extinct_[3] = {-1.1f, 1.5f, 0.f}, steps_[3] = {1.f, 16.f, 0.1f}, cutoff_[3] = {0.005f, 0.01f, 0.f};
     float vrange_[3] = {0.1f, 0.f, 1.f}, shadow_[3] = {0.8f, 1.f, 0.f};
     std::vector<float> tf_host;
+    bool tf_ramp_ = false;      // tf_host is one ramp: tf_a_ + x tf_d_
+    float tf_a_[4] = {}, tf_d_[4] = {};
     DevBuf tf_dev;
     bool tf_committed = false;
     int linear_tf(float t0, float t1, const float a[4], const float b[4]);
