@@ -925,76 +925,60 @@ __device__ inline void k_pull_body(const PullArgs& a, uint32_t bid, uint32_t) {
 }
 
 // ---------------------------------------------------- gather from buckets
-// GatherDensity without materialised subcell lists.  A voxel's value is the
-// falloff of the nearest point among those binned into its subcell; every
-// point that can raise the voxel (|p - v| < r) is binned into it, and any
-// other point gives r - |p - v| <= 0, so the nearest among all points around
-// the subcell gives the same value.  One wave per 4^3 subcell, eight per
-// 8^3 brick, with no workgroup barriers: the wave walks the buckets of the
-// (2R+1)^3 subcells around its own, keeps the points whose box reaches it
-// (staged in its own LDS list), and evaluates them row-parallel (lane =
-// 4-voxel x-row x 4 candidates per step).  The nearest point is decided on
-// float d^2, and whenever two candidates come within 2^-20 relative of each
-// other on the exact d^2 (FMA products + TwoSum), so the winner is the truly
-// nearest point (ties to the lower bucket position); its falloff is exact.
+// GatherLevelSet, and GatherDensity with accumulation, without materialised
+// subcell lists.  A voxel's value is that of the nearest point among those
+// binned into its subcell.  One wave per 4^3 subcell, eight per 8^3 brick:
+// the workgroup stages the points of the cells around the brick with the
+// subcells that list each (the reference's test), every wave lists its own
+// and evaluates them row-parallel (lane = 4-voxel x-row x 4 candidates per
+// step).  Squared distances are FP64 (vector FP64 fused multiply-adds issue
+// at the FP32 rate here): the differences are exact and d^2 is within 2 ulps
+// of 2^-53, so a plain minimum replaces a float comparison with an exact one
+// behind it for near ties, a branch that some lane of a wave took at almost
+// every candidate (level set of a 500 k slab, radius 2: 0.289 -> 0.142 ms).
 static const int GB_THREADS = 512;
-static const int GB_CHUNK = 1024;   // candidates staged per pass (two per thread)
-
-// Is candidate a (index ia) nearer to v than b (index ib)?  Accurate d^2, ties to the lower index.
-__device__ __noinline__ bool nearer_exact(float ax, float ay, float az, uint32_t ia, float bx, float by, float bz,
-                                          uint32_t ib, float vx, float vy, float vz) {
-    float ha, la, hb, lb;
-    exact_d2(ax, ay, az, vx, vy, vz, ha, la);
-    exact_d2(bx, by, bz, vx, vy, vz, hb, lb);
-    if (ha != hb) return ha < hb;
-    if (la != lb) return la < lb;
-    return ia < ib;
-}
-
-// Nearest candidate so far for one voxel: its bucket position (which also
-// fetches its coordinates when an exact comparison or the final falloff needs
-// them) and its float d^2 raised by NEAR_ULPS ulps.  Float d^2 (rounded
-// differences, two FMAs) is within 3.5 ulps of the exact value, so a candidate
-// below the raised bound may be nearer; one also below the lowered bound
-// surely is, and the few in between are settled on the exact d^2.
-static const uint32_t NEAR_ULPS = 8;
-
-struct Best {
-    float bt;       // d^2 + NEAR_ULPS ulps (INFINITY while empty)
-    uint32_t id;
-};
-
-__device__ inline void best_offer(Best& B, float d2, float px, float py, float pz, uint32_t id, float vx, float vy,
-                                  float vz, const float4* pts) {
-    if (!(d2 < B.bt)) return;
-    bool take = B.id == 0xFFFFFFFFu;
-    if (!take) {
-        const float b = __uint_as_float(__float_as_uint(B.bt) - NEAR_ULPS);
-        take = d2 < __uint_as_float(__float_as_uint(b) - NEAR_ULPS) && b > 0.0f;
-        if (!take) {
-            const float4 q = pts[B.id];
-            take = nearer_exact(px, py, pz, id, q.x, q.y, q.z, B.id, vx, vy, vz);
-        }
-    }
-    if (take) {
-        B.bt = __uint_as_float(__float_as_uint(d2) + NEAR_ULPS);
-        B.id = id;
-    }
-}
+static const int GB_CHUNK = 512;   // candidates staged per pass (one per thread)
 
 // Cell ranges of the (2 + 2R)^3 subcells around a brick and their exclusive
 // prefix (one cell per thread); returns the candidate count, 0 when the
 // brick is unreachable.
 struct GBShared {
-    uint32_t cell_off[GB_THREADS];
-    uint32_t cell_start[GB_THREADS];
-    uint16_t owner[PULL_CAP];
+    uint32_t cell_off[256];        // (2 + 2R)^3 <= 216 cells
+    uint32_t cell_start[256];
     int nbr[27];
     uint32_t wsum[GB_THREADS / 64];
-    float4 pt[GB_CHUNK];      // x, y, z, bucket position (bits)
+    double px[GB_CHUNK], py[GB_CHUNK], pz[GB_CHUNK];
     uint8_t um[GB_CHUNK];
     uint16_t lst[GB_THREADS / 64][GB_CHUNK];
 };
+
+// The cell that holds candidate f: the last one starting at or before it.
+template <class SH>
+__device__ inline int gb_cell(const SH& S, int ncell, uint32_t f) {
+    int lo = 0, hi = ncell - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (S.cell_start[mid] <= f) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// The subcells of a brick (corner `org`, two of 4 voxels per axis) whose entry
+// list holds the point: int(p - r)/4*4 <= s <= int(p + 1 + r)/4*4 on every
+// axis (C truncations; CountSubcell / InsertSubcell), p including trans.
+__device__ inline uint32_t listed_mask(const float p[3], float r, const int org[3]) {
+    uint32_t am[3], um = 0;
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++) {
+        const int lo = child_cell(int(p[ax] - r), 2) * 4, hi = child_cell(int(p[ax] + 1 + r), 2) * 4;
+        am[ax] = (lo <= org[ax] && org[ax] <= hi ? 1u : 0u) | (lo <= org[ax] + 4 && org[ax] + 4 <= hi ? 2u : 0u);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+        if ((am[0] >> (k & 1)) & (am[1] >> ((k >> 1) & 1)) & (am[2] >> (k >> 2)) & 1u) um |= 1u << k;
+    return um;
+}
 
 // The brick's 27 neighbour ids, one per thread below 27 (loaded by the
 // caller ahead of its own checks, so the load overlaps them).
@@ -1040,6 +1024,14 @@ __device__ inline uint32_t gb_setup(int R, int nb_mine, const uint32_t* bcnt, co
     return total;
 }
 
+// The smaller of two doubles that are no NaNs (fmin quiets its operands first,
+// an instruction each).
+__device__ inline double min_f64(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
 template <typename AT>
 __device__ inline void k_bucket_gather_body(const BucketGatherArgs& a, uint32_t bid, uint32_t) {
     __shared__ GBShared S;
@@ -1051,116 +1043,94 @@ __device__ inline void k_bucket_gather_body(const BucketGatherArgs& a, uint32_t 
     const float r = a.radius;
     const int R = a.R, span = 2 + 2 * R, ncell = span * span * span;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int row = lane & 15, g = lane >> 4;
-    const int ry = row & 3, rz = row >> 2;
+    // lane: two 4-voxel x-rows (y = ry, ry + 1) of layer rz, every 8th candidate
+    const int ry = (lane & 1) * 2, rz = (lane >> 1) & 3, g = lane >> 3;
     // this wave's subcell (x fastest, as CalcSubcellPos numbers them)
     const int sx = bn->mPos[0] + (wave & 1) * 4, sy = bn->mPos[1] + ((wave >> 1) & 1) * 4,
               sz = bn->mPos[2] + (wave >> 2) * 4;
-    const float fx[4] = {float(sx), float(sx + 1), float(sx + 2), float(sx + 3)};
-    const float fy = float(sy + ry), fz = float(sz + rz);
-    Best B[4];
+    const double fx = double(sx), fy = double(sy + ry), fz = double(sz + rz);
+    double B[2][4];      // least squared distance per voxel
 #pragma unroll
-    for (int x = 0; x < 4; x++) B[x] = Best{INFINITY, 0xFFFFFFFFu};
+    for (int k = 0; k < 8; k++) B[k >> 2][k & 3] = INFINITY;
     const uint32_t T = gb_setup(R, gb_nbr(a.nbr, brick), a.bcnt, a.boff, S);
     __syncthreads();
     const int org[3] = {bn->mPos[0], bn->mPos[1], bn->mPos[2]};
     const u64 lower = lane ? ((~0ull) >> (64 - lane)) : 0ull;
-    for (uint32_t w0 = 0; w0 < T; w0 += PULL_CAP) {
-        // cell of every candidate in the window
-        for (int c = threadIdx.x; c < ncell; c += GB_THREADS) {
-            uint32_t beg = S.cell_start[c];
-            uint32_t end = (c + 1 < ncell) ? S.cell_start[c + 1] : T;
-            for (uint32_t f = max(beg, w0); f < end && f < w0 + PULL_CAP; f++) S.owner[f - w0] = uint16_t(c);
+    for (uint32_t c0 = 0; c0 < T; c0 += GB_CHUNK) {
+        // candidates of this chunk: positions and the subcells of the brick that list each
+        const uint32_t nc = min(uint32_t(GB_CHUNK), T - c0);
+        if (c0) __syncthreads();
+        const int q = threadIdx.x;
+        uint32_t um = 0;
+        if (uint32_t(q) < nc) {
+            const uint32_t f = c0 + uint32_t(q);
+            const int c = gb_cell(S, ncell, f);
+            const float4 p = a.sorted[S.cell_off[c] + (f - S.cell_start[c])];
+            const float pp[3] = {p.x, p.y, p.z};
+            um = listed_mask(pp, r, org);
+            S.px[q] = p.x;
+            S.py[q] = p.y;
+            S.pz[q] = p.z;
         }
+        S.um[q] = uint8_t(um);
         __syncthreads();
-        const uint32_t wend = min(T, w0 + PULL_CAP);
-        for (uint32_t c0 = w0; c0 < wend; c0 += GB_CHUNK) {
-            // candidates of this chunk: positions and the subcells of the brick each can reach
-            for (int q = threadIdx.x; q < GB_CHUNK; q += GB_THREADS) {
-                const uint32_t f = c0 + q;
-                uint32_t um = 0;
-                if (f < wend) {
-                    const int c = S.owner[f - w0];
-                    const uint32_t pos = S.cell_off[c] + (f - S.cell_start[c]);
-                    const float4 p = a.sorted[pos];
-                    const float pp[3] = {p.x, p.y, p.z};
-                    uint32_t am[3];
-#pragma unroll
-                    for (int ax = 0; ax < 3; ax++) {
-                        // the entry-list test of CountSubcell/InsertSubcell: subcell
-                        // origin s is listed when int(p - r)/4*4 <= s <= int(p + 1 + r)/4*4
-                        // (C truncations), p including trans as bucketed
-                        const int lo = child_cell(int(pp[ax] - r), 2) * 4, hi = child_cell(int(pp[ax] + 1 + r), 2) * 4;
-                        am[ax] = (lo <= org[ax] && org[ax] <= hi ? 1u : 0u) |
-                                 (lo <= org[ax] + 4 && org[ax] + 4 <= hi ? 2u : 0u);
-                    }
-#pragma unroll
-                    for (int k = 0; k < 8; k++)
-                        if ((am[0] >> (k & 1)) & (am[1] >> ((k >> 1) & 1)) & (am[2] >> (k >> 2)) & 1u) um |= 1u << k;
-                    S.pt[q] = make_float4(p.x, p.y, p.z, __uint_as_float(pos));
-                }
-                S.um[q] = uint8_t(um);
-            }
-            __syncthreads();
-            // this wave's candidates, in candidate order
-            uint32_t n = 0;
-            const int ngrp = int((min(uint32_t(GB_CHUNK), wend - c0) + 63) / 64);
-            for (int grp = 0; grp < ngrp; grp++) {
-                const bool on = (S.um[grp * 64 + lane] >> wave) & 1u;
-                const u64 bal = __ballot(on);
-                if (on) S.lst[wave][n + uint32_t(__popcll(bal & lower))] = uint16_t(grp * 64 + lane);
-                n += uint32_t(__popcll(bal));
-            }
-            __builtin_amdgcn_wave_barrier();
-            for (uint32_t k = 0; k < n; k += 4) {
-                const uint32_t j = k + uint32_t(g);
-                if (j < n) {
-                    const float4 pe = S.pt[S.lst[wave][j]];
-                    const float px = pe.x, py = pe.y, pz = pe.z;
-                    const uint32_t id = __float_as_uint(pe.w);
-                    const float dy = py - fy, dz = pz - fz;
-                    const float dyz = __builtin_fmaf(dy, dy, dz * dz);
-#pragma unroll
-                    for (int x = 0; x < 4; x++) {
-                        const float dx = px - fx[x];
-                        best_offer(B[x], __builtin_fmaf(dx, dx, dyz), px, py, pz, id, fx[x], fy, fz, a.sorted);
-                    }
-                }
-            }
-            __syncthreads();
+        // this wave's candidates, in candidate order
+        uint32_t n = 0;
+        for (uint32_t k = 0; k < nc; k += 64) {
+            const bool on = (S.um[k + uint32_t(lane)] >> wave) & 1u;
+            const u64 bal = __ballot(on);
+            if (on) S.lst[wave][n + uint32_t(__popcll(bal & lower))] = uint16_t(k + uint32_t(lane));
+            n += uint32_t(__popcll(bal));
         }
-    }
-    // merge the four candidate groups of each row
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t k = 0; k < n; k += 8) {
+            // (past the end: the last candidate again)
+            const int c = S.lst[wave][min(k + uint32_t(g), n - 1)];
+            const double dx = S.px[c] - fx, dy = S.py[c] - fy, dz = S.pz[c] - fz;
+            const double z2 = dz * dz, d1 = dy - 1.0;
+            const double yz[2] = {__builtin_fma(dy, dy, z2), __builtin_fma(d1, d1, z2)};
 #pragma unroll
-    for (int sh = 16; sh <= 32; sh <<= 1) {
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-            const float obt = __shfl_xor(B[x].bt, sh, 64);
-            const uint32_t oi = __shfl_xor(B[x].id, sh, 64);
-            if (oi != 0xFFFFFFFFu) {
-                const float4 q = a.sorted[oi];
-                best_offer(B[x], __uint_as_float(__float_as_uint(obt) - NEAR_ULPS), q.x, q.y, q.z, oi, fx[x], fy, fz,
-                           a.sorted);
+            for (int x = 0; x < 4; x++) {
+                const double e = dx - double(x);
+                B[0][x] = min_f64(B[0][x], __builtin_fma(e, e, yz[0]));
+                B[1][x] = min_f64(B[1][x], __builtin_fma(e, e, yz[1]));
             }
         }
     }
-    if (g != 0) return;
+    // merge the eight candidate groups of each row
+#pragma unroll
+    for (int sh = 8; sh <= 32; sh <<= 1)
+#pragma unroll
+        for (int k = 0; k < 8; k++) B[k >> 2][k & 3] = min_f64(B[k >> 2][k & 3], __shfl_xor(B[k >> 2][k & 3], sh, 64));
+    // lane group g writes voxel x = g & 3 of row g >> 2
     AT* atlas = reinterpret_cast<AT*>(a.atlas);
-    const int vy = sy + ry, vz = sz + rz;
-    const u64 aoff = atlas_offset(t, bn->mValue[0] + (sx - bn->mPos[0]), bn->mValue[1] + (vy - bn->mPos[1]),
-                                  bn->mValue[2] + (vz - bn->mPos[2]));
+    double D = INFINITY;
 #pragma unroll
-    for (int x = 0; x < 4; x++) {
-        float val = a.accumulate ? load_atlas<AT>(atlas, aoff + x) : (a.levelset ? 3.0f : 0.0f);
-        if (B[x].id != 0xFFFFFFFFu) {
-            const float4 q = a.sorted[B[x].id];
-            const float f = falloff_accurate(q.x, q.y, q.z, sx + x, vy, vz, r);
-            val = a.levelset ? fminf(val, -f) : fmaxf(val, f);
-        }
-        store_atlas<AT>(atlas, aoff + x, val);
+    for (int k = 0; k < 8; k++)
+        if (g == k) D = B[k >> 2][k & 3];
+    const int vx = sx + (g & 3), vy = sy + ry + (g >> 2), vz = sz + rz;
+    const u64 aoff = atlas_offset(t, bn->mValue[0] + (vx - bn->mPos[0]), bn->mValue[1] + (vy - bn->mPos[1]),
+                                  bn->mValue[2] + (vz - bn->mPos[2]));
+    float val = a.accumulate ? load_atlas<AT>(atlas, aoff) : (a.levelset ? 3.0f : 0.0f);
+    if (D < INFINITY) {
+        const float d = float(sqrt(D) - double(r));
+        val = a.levelset ? fminf(val, d) : fmaxf(val, -d);
     }
+    store_atlas<AT>(atlas, aoff, val);
 }
-GVDB_MULTI_T(k_bucket_gather, typename AT, AT, BucketGatherArgs, GB_THREADS)
+// Written out to ask for eight waves per SIMD (four workgroups per CU).
+template <typename AT>
+__global__ __launch_bounds__(GB_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bucket_gather(
+    BucketGatherArgs a0, MultiMap m) {
+    const uint32_t bi = m.xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    if (m.G <= 1) {
+        k_bucket_gather_body<AT>(a0, bi, gridDim.x);
+        return;
+    }
+    const int g = multi_grid(m, bi);
+    const uint32_t* first = multi_first(m);
+    k_bucket_gather_body<AT>(multi_rec<BucketGatherArgs>(m, g), bi - first[g], first[g + 1] - first[g]);
+}
 
 // GatherDensity by scattering: every candidate point offers itself to the
 // voxels of the brick within the radius of it, in a copy of the brick held
@@ -1562,16 +1532,22 @@ hipError_t launch_bucket_gather_multi(const BucketGatherArgs* a, int G, Arena* a
 // (old + sum) / (count + 1), in integer division: the mean of the list's
 // colours, independent of the order the entries were inserted in (the
 // reference adds floats in atomic-insertion order).  One workgroup per brick
-// reads the candidates of the brick's (2 + 2R)^3 cells, as the density
-// gather does, and counts a candidate for each of the brick's subcells whose
-// list the insert rule puts it in: int(w - r)/sc*sc <= s <= int(w + 1 + r)/sc*sc
-// on every axis (kernels/cuda_gvdb_particles.cuh:237-242).
-static const int CG_THREADS = 256;
+// stages the candidates of the brick's (2 + 2R)^3 cells with the subcells
+// whose list the insert rule puts each in: int(w - r)/sc*sc <= s <=
+// int(w + 1 + r)/sc*sc on every axis (kernels/cuda_gvdb_particles.cuh:237-242);
+// then one wave per subcell adds up its own, 64 candidates a step in two
+// packed words, and reduces once (adding every candidate to its subcells'
+// five counters by LDS atomics queued the whole workgroup on 40 addresses:
+// 250 k points of a shell, with the density gather, 0.217 -> 0.090 ms).
+static const int CG_THREADS = 256;   // four waves, two subcells each
+static const int CG_CHUNK = 512;
 struct CGShared {
-    uint32_t cell_off[CG_THREADS];
-    uint32_t cell_start[CG_THREADS];
+    uint32_t cell_off[256];
+    uint32_t cell_start[256];
     int nbr[27];
     uint32_t wsum[CG_THREADS / 64];
+    uint32_t clr[CG_CHUNK];
+    uint8_t um[CG_CHUNK];
     uint32_t sum[8][5];   // r, g, b, a, entries per subcell of the brick
 };
 
@@ -1583,46 +1559,56 @@ __device__ inline void k_gather_color_body(const ColorArgs& a, uint32_t bid, uin
     const int nb_mine = gb_nbr(a.nbr, brick);
     if (bn->mParent == ID_UNDEF64) return;        // unlinked leaves have no subcells
     if (!bn->mFlags || bn->mValue[0] < 0) return;  // no atlas slot to write (uniform per brick)
-    const int tid = threadIdx.x;
-    if (tid < 40) (&S.sum[0][0])[tid] = 0;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t T = gb_setup<CG_THREADS>(a.R, nb_mine, a.bcnt, a.boff, S);
     __syncthreads();
     const int span = 2 + 2 * a.R, ncell = span * span * span;
-    const int sc = a.scs, sd = t.brickwid / sc;   // subcells per axis (2 for 8^3 bricks, sc 4)
     const float r = a.radius;
-    for (uint32_t f = uint32_t(tid); f < T; f += CG_THREADS) {
-        int lo = 0, hi = ncell - 1;                // last cell starting at or before f
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (S.cell_start[mid] <= f) lo = mid;
-            else hi = mid - 1;
+    const int org[3] = {bn->mPos[0], bn->mPos[1], bn->mPos[2]};
+    uint32_t acc[2][5] = {};
+    for (uint32_t c0 = 0; c0 < T; c0 += CG_CHUNK) {
+        const uint32_t nc = min(uint32_t(CG_CHUNK), T - c0);
+        if (c0) __syncthreads();                    // the previous chunk is added up
+        for (uint32_t q = uint32_t(tid); q < nc; q += CG_THREADS) {
+            const uint32_t f = c0 + q;
+            const int c = gb_cell(S, ncell, f);
+            const float4 p = a.sorted[S.cell_off[c] + (f - S.cell_start[c])];
+            const float pp[3] = {p.x, p.y, p.z};
+            S.um[q] = uint8_t(listed_mask(pp, r, org));
+            S.clr[q] = __float_as_uint(p.w);
         }
-        const float4 q = a.sorted[S.cell_off[lo] + (f - S.cell_start[lo])];
-        const float w[3] = {q.x, q.y, q.z};
-        uint32_t m[3];                              // subcells of the brick along each axis whose list takes it
-        for (int ax = 0; ax < 3; ax++) {
-            const int s0 = int(w[ax] - r) / sc * sc, s1 = int(w[ax] + 1.0f + r) / sc * sc;
-            m[ax] = 0;
-            for (int k = 0; k < sd; k++) {
-                const int st = bn->mPos[ax] + k * sc;
-                if (s0 <= st && st <= s1) m[ax] |= 1u << k;
+        __syncthreads();
+        // at most 8 candidates a lane and chunk: the packed sums stay below 2^16
+        uint32_t rb[2] = {0, 0}, ga[2] = {0, 0}, n[2] = {0, 0};
+        for (uint32_t q = uint32_t(lane); q < nc; q += 64) {
+            const uint32_t u = S.um[q] >> wave, c = S.clr[q];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const uint32_t on = (u >> (4 * h)) & 1u, k = on ? c : 0u;
+                rb[h] += k & 0x00FF00FFu;
+                ga[h] += (k >> 8) & 0x00FF00FFu;
+                n[h] += on;
             }
         }
-        if (!(m[0] && m[1] && m[2])) continue;
-        const uint32_t c = __float_as_uint(q.w);
-        for (int kz = 0; kz < sd; kz++)
-            for (int ky = 0; ky < sd; ky++)
-                for (int kx = 0; kx < sd; kx++) {
-                    if (!((m[0] >> kx) & (m[1] >> ky) & (m[2] >> kz) & 1u)) continue;
-                    uint32_t* sm = S.sum[(kz * sd + ky) * sd + kx];
-                    atomicAdd(sm + 0, c & 0xFFu);
-                    atomicAdd(sm + 1, (c >> 8) & 0xFFu);
-                    atomicAdd(sm + 2, (c >> 16) & 0xFFu);
-                    atomicAdd(sm + 3, c >> 24);
-                    atomicAdd(sm + 4, 1u);
-                }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            acc[h][0] += rb[h] & 0xFFFFu;
+            acc[h][1] += ga[h] & 0xFFFFu;
+            acc[h][2] += rb[h] >> 16;
+            acc[h][3] += ga[h] >> 16;
+            acc[h][4] += n[h];
+        }
     }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int k = 0; k < 5; k++) {
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) acc[h][k] += __shfl_xor(acc[h][k], d, 64);
+            if (lane == 0) S.sum[wave + 4 * h][k] = acc[h][k];
+        }
     __syncthreads();
+    const int sc = 4, sd = 2;
     uint32_t* atlas = reinterpret_cast<uint32_t*>(a.atlas) + slot_of(t, bn->mValue) * u64(t.brick_vox);
     const int w = t.brickwid, pbr = t.brick_res, ap = t.apron;
     for (int v = tid; v < w * w * w; v += CG_THREADS) {
@@ -1648,9 +1634,8 @@ GVDB_MULTI(k_gather_color, ColorArgs, CG_THREADS)
 hipError_t launch_gather_color_multi(const ColorArgs* a, int G, Arena* ar, hipStream_t s) {
     std::vector<uint32_t> nb(G);
     for (int g = 0; g < G; g++) {
-        if (a[g].t.res[0] != 8 || a[g].R < 1 || a[g].R > 2 || a[g].scs <= 0 || a[g].t.brickwid % a[g].scs ||
-            a[g].t.brickwid / a[g].scs > 2 || (2 + 2 * a[g].R) * (2 + 2 * a[g].R) * (2 + 2 * a[g].R) > CG_THREADS)
-            return hipErrorInvalidValue;
+        // 8^3 bricks of 4^3 subcells; a cell per thread
+        if (a[g].t.res[0] != 8 || a[g].scs != 4 || a[g].R < 1 || a[g].R > 2) return hipErrorInvalidValue;
         nb[g] = uint32_t(a[g].nleaves > 0 ? a[g].nleaves : 0);
     }
     MultiLaunch L;
