@@ -33,6 +33,11 @@ __device__ inline void k_neighbors_body(const NbrArgs& a, uint32_t bid, uint32_t
     const int b = int(g >> 5), d = int(g & 31);
     const bool valid = b < a.n && d < 27;
     int v = -1;
+    if (a.bcnt) {
+        if (b < a.n && d < a.spb) a.bcnt[u64(b) * u64(a.spb) + u64(d)] = 0;
+        if (g < 64) a.lenparts[g] = 0;
+        if (g == 0) *a.orphans = 0;
+    }
     if (valid) {
         const Node* n = t.nodes[0] + b;
         int dx, dy, dz;

@@ -29,6 +29,13 @@ struct BitDomain {
     u64 nwords;   // 32-bit words
 };
 
+// A result word that the host may read from its own (pinned) memory after it
+// has waited for an event or the stream: stored at system scope.
+template <class T>
+__device__ inline void store_word(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---- utilities (util.hip)
 struct FillArgs {
     void* p;
@@ -65,12 +72,12 @@ hipError_t launch_scan_u32(const uint32_t* in0, const uint32_t* in1, int mode, u
 struct BboxArgs {
     PointSrc pts;
     float o[3];
-    uint32_t* keys6;      // orderable float keys: min x,y,z then max x,y,z
-    uint32_t* part;       // BBOX_PART_WORDS: six keys per block
+    uint32_t* keys7;      // orderable float keys: min x,y,z then max x,y,z; then 1 if a coordinate was no finite number
+    uint32_t* part;       // BBOX_PART_WORDS: the seven words per block
     uint32_t nparts;      // set by the launcher: blocks of the grid
 };
 static const int BBOX_BLOCKS = 2048;                         // blocks per grid at most
-static const int BBOX_PART_WORDS = BBOX_BLOCKS * 6;
+static const int BBOX_PART_WORDS = BBOX_BLOCKS * 7;
 hipError_t launch_bbox_multi(const BboxArgs* a, int G, Arena* ar, hipStream_t s);
 
 struct MarkArgs {
@@ -86,7 +93,23 @@ struct MarkArgs {
     uint32_t* masks;      // optional zeroed u32 per level-0 domain brick
     uint8_t* bytes;       // optional zeroed byte per domain brick: A at 0, B at nwords * 32 (instead of masks)
 };
-hipError_t launch_mark_points_multi(const MarkArgs* a, int G, Arena* ar, hipStream_t s);
+// pack: byte marks go on to the bitmaps (otherwise launch_box_levels_multi reads them)
+hipError_t launch_mark_points_multi(const MarkArgs* a, int G, Arena* ar, hipStream_t s, bool pack);
+
+// Byte marks to every level's bitmaps, ranks and counts in one workgroup, for
+// boxes whose bitmaps take at most BOX_WORDS words in all.
+static const uint32_t BOX_WORDS = 15360;
+static const int BOX_LEVELS = 5;
+struct BoxArgs {
+    const uint8_t* bytes;
+    int dilate, D;                // D <= BOX_LEVELS
+    BitDomain dom[BOX_LEVELS];
+    int logdim[BOX_LEVELS];
+    uint32_t* bitmaps;            // per level: A, then B when dilating
+    uint32_t* ranks;              // the same layout
+    uint32_t* counts;             // [2 L + set]
+};
+hipError_t launch_box_levels_multi(const BoxArgs* a, int G, Arena* ar, hipStream_t s);
 
 struct ParentArgs {
     BitDomain dc;
@@ -110,11 +133,19 @@ struct LevelBuild {
     int lev;
     int range;
 };
+struct RootArgs {
+    Node* root;
+    int pos[3];
+    int lev;
+};
 struct EmitArgs {
     LevelBuild L;
     Node* nodes;
     int has_clist;
     u64* btab;            // optional (level 0, box up to BRICK_TAB_MAX bits): the brick table
+    u64* fill;            // child lists to empty, fill_n entries
+    u64 fill_n;
+    RootArgs root;        // root.root: also the root node (level 0's record)
 };
 hipError_t launch_emit_nodes_multi(const EmitArgs* a, int G, Arena* ar, hipStream_t s);
 
@@ -168,11 +199,6 @@ hipError_t launch_emit_list(const KeyLevel& L, Node* nodes, int has_clist, hipSt
 hipError_t launch_link_list(const KeyLevel& C, const KeyLevel& P, int parent_is_root, int ld, Node* cnodes,
                             u64* pclists, u64 clist_len, hipStream_t s);
 
-struct RootArgs {
-    Node* root;
-    int pos[3];
-    int lev;
-};
 hipError_t launch_write_root_multi(const RootArgs* a, int G, Arena* ar, hipStream_t s);
 
 // ---- incremental topology (ActivateIncreBricksGPU, topology.hip)
@@ -230,10 +256,14 @@ struct ComputeArgs {
 hipError_t launch_compute(const ComputeArgs& a, hipStream_t s);
 
 // ---- atlas & points (points.hip)
+// slot_scan == nullptr: every leaf is in use, leaf i takes slot i and the
+// launch also clears the map's entries n .. map_n - 1 (otherwise the map is
+// cleared beforehand and map_n is 0).
 struct AtlasArgs {
     Tree t;
     const uint32_t* slot_scan;
     int n;
+    int map_n;
 };
 hipError_t launch_update_atlas_multi(const AtlasArgs* a, int G, Arena* ar, hipStream_t s);
 
@@ -244,6 +274,7 @@ struct FlagArgs {
     int n;
     int mode;
 };
+hipError_t launch_iota(uint32_t* out, u64 n, hipStream_t s);   // out[i] = i
 hipError_t launch_leaf_flags_multi(const FlagArgs* a, int G, Arena* ar, hipStream_t s);
 
 // ComputeBounds over flagged leaves: out6 = min corner, max corner + range
@@ -328,7 +359,13 @@ struct BucketArgs {
     int rule;             // BIN_FLOAT or BIN_FP16
     BrickTab bt;          // leaf lookup (tab == nullptr: the walk)
 };
-hipError_t launch_sum_parts_multi(const u64* const* parts, u64* const* out, int G, Arena* ar, hipStream_t s);
+struct SumArgs {
+    const u64* parts;
+    u64* out;
+    const uint32_t* orphans;
+    uint32_t* orphans_out;   // or null
+};
+hipError_t launch_sum_parts_multi(const SumArgs* a, int G, Arena* ar, hipStream_t s);
 hipError_t launch_bucket_points_multi(const BucketArgs* a, int G, Arena* ar, hipStream_t s);
 
 struct ScatterArgs {
@@ -416,6 +453,12 @@ struct NbrArgs {
     uint32_t* mask;       // optional: bit d set when nbr[b*27 + d] >= 0 (written whole)
     long long* base;      // optional: atlas offset of each neighbour's brick (d = 13: own), -1 if none
     BrickTab bt;          // leaf lookup (tab == nullptr: the walks)
+    // optional (an insert follows): the brick's spb bucket counters, the 64
+    // partial entry counts and the orphan count, set to zero
+    uint32_t* bcnt;
+    int spb;
+    u64* lenparts;
+    uint32_t* orphans;
 };
 hipError_t launch_neighbors_multi(const NbrArgs* a, int G, Arena* ar, hipStream_t s);
 

@@ -44,6 +44,13 @@ static int drain(Volume* v, const Exec& ex, int G) {
     return GVDB_OK;
 }
 
+// Waits for kernels that wrote their results to host memory themselves.
+static int wait_host(Volume* v, const Exec& ex) {
+    XCHK(v, hipStreamSynchronize(ex.s));
+    if (ex.ar) ex.ar->reset();
+    return GVDB_OK;
+}
+
 #define FAILG(g, code)               \
     do {                             \
         if (failed) *failed = (g);   \
@@ -71,11 +78,12 @@ int Volume::multi_rebuild_topology(Volume* const* vs, int G, const int* n, const
         PointSrc P = vs[g]->pts_;
         P.n = n[g];
         XCHK(vs[g], vs[g]->bbox_part_.ensure(size_t(BBOX_PART_WORDS) * 4));
-        ba[g] = BboxArgs{P, {orig3[3 * g], orig3[3 * g + 1], orig3[3 * g + 2]}, ex.dsmall + g * SMALL_WORDS + SM_BBOX,
+        // straight to host memory: nothing on the device reads the keys
+        ba[g] = BboxArgs{P, {orig3[3 * g], orig3[3 * g + 1], orig3[3 * g + 2]}, ex.hsmall + g * SMALL_WORDS + SM_BBOX,
                          vs[g]->bbox_part_.as<uint32_t>()};
     }
     XCHK(v0, launch_bbox_multi(ba.data(), G, ex.ar, ex.s));
-    int rc = drain(v0, ex, G);
+    int rc = wait_host(v0, ex);
     if (rc) return rc;
 
     // per grid: bounds, depth and the reference's choice between a full and
@@ -87,9 +95,11 @@ int Volume::multi_rebuild_topology(Volume* const* vs, int G, const int* n, const
     // would walk a tree of another depth.
     std::vector<float> mnmx(6 * size_t(G));
     std::vector<int> depth(G), root(3 * size_t(G)), full_idx;
+    std::vector<uint8_t> odd(G);
     for (int g = 0; g < G; g++) {
         Volume* v = vs[g];
         const uint32_t* hk = ex.hsmall + g * SMALL_WORDS + SM_BBOX;
+        odd[g] = hk[6] != 0;
         for (int a = 0; a < 3; a++) {
             mnmx[6 * g + a] = key_float(hk[a]);
             mnmx[6 * g + 3 + a] = key_float(hk[3 + a]);
@@ -137,6 +147,7 @@ int Volume::multi_rebuild_topology(Volume* const* vs, int G, const int* n, const
             const Exec eg{ex.s, ex.ar, ex.dsmall + g * SMALL_WORDS, ex.hsmall + g * SMALL_WORDS};
             rc = v->keyed_build(n[g], radius[g], orig3 + 3 * g, depth[g], &root[3 * g], dom, eg);
             if (rc) FAILG(g, rc);
+            v->note_full_build(&mnmx[6 * g], odd[g] != 0, radius[g], dom[0]);
         }
         full_idx.swap(bitmap_idx);
     }
@@ -145,17 +156,20 @@ int Volume::multi_rebuild_topology(Volume* const* vs, int G, const int* n, const
         std::vector<Volume*> fv(F);
         std::vector<int> fn(F), fd(F), fr(3 * size_t(F));
         std::vector<float> frad(F), fo(3 * size_t(F)), fm(6 * size_t(F));
+        std::vector<uint8_t> fodd(F);
         for (int k = 0; k < F; k++) {
             const int g = full_idx[k];
             fv[k] = vs[g];
             fn[k] = n[g];
             fd[k] = depth[g];
             frad[k] = radius[g];
+            fodd[k] = odd[g];
             for (int a = 0; a < 3; a++) { fr[3 * k + a] = root[3 * g + a]; fo[3 * k + a] = orig3[3 * g + a]; }
             for (int a = 0; a < 6; a++) fm[6 * k + a] = mnmx[6 * g + a];
         }
         int f = -1;
-        rc = multi_full_build(fv.data(), F, fn.data(), frad.data(), fo.data(), fd.data(), fr.data(), fm.data(), ex, &f);
+        rc = multi_full_build(fv.data(), F, fn.data(), frad.data(), fo.data(), fd.data(), fr.data(), fm.data(), fodd.data(),
+                              ex, &f);
         if (rc) {
             if (failed && f >= 0) *failed = full_idx[f];
             return rc;
@@ -196,6 +210,30 @@ bool Volume::plan_domains(const Volume* v, int D, const int rootPos[3], const fl
     return true;
 }
 
+// After a full build: its leaves, and their box.  A point's bricks are its own
+// and those of [int(w) - r, int(w) + 2r], clipped to the build's box; each is
+// a non-decreasing function of the coordinate, so the ends of the leaves' box
+// on an axis come from the least and the greatest coordinate there, when every
+// point counted (all finite and none negative).
+void Volume::note_full_build(const float* mnmx, bool odd, float radius, const BitDomain& d0) {
+    full_gen_ = topo_gen_;
+    full_box_ = !odd && mnmx[0] >= 0.0f && mnmx[1] >= 0.0f && mnmx[2] >= 0.0f;
+    const int range0 = int(range_[0]);
+    const float inv = 1.0f / float(range0);
+    for (int a = 0; a < 3 && full_box_; a++) {
+        const float mn = mnmx[a], mx = mnmx[3 + a];
+        int lo = int(floorf(mn * inv)), hi = int(floorf(mx * inv));
+        if (radius >= 1.0f) {
+            lo = std::min(lo, int(float(int(mn)) - radius) / range0);
+            hi = std::max(hi, int(float(int(mx)) + 2.0f * radius) / range0);
+        }
+        lo = std::max(lo, d0.lo[a]);
+        hi = std::min(hi, d0.lo[a] + d0.dim[a] - 1);
+        full_min_[a] = float(lo * range0);
+        full_max_[a] = float(hi * range0 + range0);
+    }
+}
+
 // Level-0 boxes above this many bricks take the keyed build (bitmaps of
 // 2^34 bits are 2 GiB per level and set).
 static const u64 BITMAP_MAX_BITS = u64(1) << 34;
@@ -205,7 +243,8 @@ static bool keyed_build_wanted(const BitDomain& d0) { return d0.nbits > BITMAP_M
 // The full build of RebuildTopology (ActivateBricksGPU + ActivateExtraBricksGPU)
 // for grids already cleared, with their depth, root corner and point bounds.
 int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float* radius, const float* orig3,
-                             const int* depth, const int* rootPos, const float* mnmx, const Exec& ex, int* failed) {
+                             const int* depth, const int* rootPos, const float* mnmx, const uint8_t* odd, const Exec& ex,
+                             int* failed) {
     Volume* v0 = vs[0];
     int rc = 0;
     // per grid: depth, root, domains, scratch
@@ -218,9 +257,13 @@ int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float
         uint32_t* masks = nullptr;
         uint8_t* bytes = nullptr;
         bool btab = false;
+        u64 bm_words = 0;
     };
     std::vector<Plan> plan(G);
     std::vector<FillArgs> fills;
+    // every grid of the call on byte marks and in a small box: its levels in
+    // one workgroup (k_box_levels)
+    bool boxed = true;
     for (int g = 0; g < G; g++) {
         Volume* v = vs[g];
         Plan& pl = plan[g];
@@ -249,7 +292,7 @@ int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float
         XCHK(v, v->bitmaps_.ensure(bm_words * 4 + 256));
         XCHK(v, v->ranks_.ensure(rk_words * 4 + 256));
         XCHK(v, v->scan_tmp_.ensure(tmp_words * 4 + 256));
-        fills.push_back(FillArgs{v->bitmaps_.p, bm_words, 0, 0});
+        pl.bm_words = bm_words;
         // marks: a byte per domain brick (own-brick marks, then dilation
         // marks, whole 32-byte groups) up to 2^27 bricks; else direction masks
         // (4 bytes per domain brick) while that stays comparable to the point
@@ -272,7 +315,10 @@ int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float
             pl.masks = v->masks_.as<uint32_t>();
             fills.push_back(FillArgs{pl.masks, pl.dom[0].nbits, 0, 0});
         }
+        boxed = boxed && path == 1 && pl.bm_words <= BOX_WORDS && D <= BOX_LEVELS;
     }
+    if (!boxed)
+        for (int g = 0; g < G; g++) fills.push_back(FillArgs{vs[g]->bitmaps_.p, plan[g].bm_words, 0, 0});
     XCHK(v0, launch_fill_multi(fills.data(), int(fills.size()), ex.ar, ex.s));
     auto A = [&](int g, int L) { return vs[g]->bitmaps_.as<uint32_t>() + plan[g].bm_off[L]; };
     auto B = [&](int g, int L) {
@@ -289,37 +335,55 @@ int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float
                          plan[g].bytes};
         maxD = std::max(maxD, plan[g].D);
     }
-    XCHK(v0, launch_mark_points_multi(ma.data(), G, ex.ar, ex.s));
-    for (int L = 1; L < maxD; L++) {
-        std::vector<ParentArgs> pa;
-        for (int g = 0; g < G; g++)
-            if (L < plan[g].D)
-                pa.push_back(ParentArgs{plan[g].dom[L - 1], A(g, L - 1), B(g, L - 1), vs[g]->logdim_[L], plan[g].dom[L],
-                                        A(g, L), B(g, L)});
-        XCHK(v0, launch_mark_parents_multi(pa.data(), int(pa.size()), ex.ar, ex.s));
-    }
-    std::vector<ScanArgs> sa;
-    for (int g = 0; g < G; g++) {
-        Volume* v = vs[g];
-        uint32_t* rk = v->ranks_.as<uint32_t>();
-        uint32_t* tmp = v->scan_tmp_.as<uint32_t>();
-        uint32_t* counts = ex.dsmall + g * SMALL_WORDS + SM_COUNTS;
-        for (int L = 0; L < plan[g].D; L++) {
-            const BitDomain& d = plan[g].dom[L];
-            sa.push_back(ScanArgs{A(g, L), nullptr, 1, rk + plan[g].rk_off[L], d.nwords, tmp + plan[g].tmp_off[2 * L],
-                                  counts + 2 * L});
-            if (plan[g].dilate)
-                sa.push_back(ScanArgs{A(g, L), B(g, L), 2, rk + plan[g].rk_off[L] + d.nwords, d.nwords,
-                                      tmp + plan[g].tmp_off[2 * L + 1], counts + 2 * L + 1});
+    XCHK(v0, launch_mark_points_multi(ma.data(), G, ex.ar, ex.s, !boxed));
+    // the counts go straight to host memory
+    auto counts = [&](int g) { return ex.hsmall + g * SMALL_WORDS + SM_COUNTS; };
+    if (boxed) {
+        std::vector<BoxArgs> bx(G);
+        for (int g = 0; g < G; g++) {
+            Volume* v = vs[g];
+            BoxArgs& b = bx[g];
+            b.bytes = plan[g].bytes;
+            b.dilate = plan[g].dilate ? 1 : 0;
+            b.D = plan[g].D;
+            for (int L = 0; L < plan[g].D; L++) {
+                b.dom[L] = plan[g].dom[L];
+                b.logdim[L] = v->logdim_[L];
+            }
+            b.bitmaps = v->bitmaps_.as<uint32_t>();
+            b.ranks = v->ranks_.as<uint32_t>();
+            b.counts = counts(g);
         }
+        XCHK(v0, launch_box_levels_multi(bx.data(), G, ex.ar, ex.s));
+    } else {
+        for (int L = 1; L < maxD; L++) {
+            std::vector<ParentArgs> pa;
+            for (int g = 0; g < G; g++)
+                if (L < plan[g].D)
+                    pa.push_back(ParentArgs{plan[g].dom[L - 1], A(g, L - 1), B(g, L - 1), vs[g]->logdim_[L],
+                                            plan[g].dom[L], A(g, L), B(g, L)});
+            XCHK(v0, launch_mark_parents_multi(pa.data(), int(pa.size()), ex.ar, ex.s));
+        }
+        std::vector<ScanArgs> sa;
+        for (int g = 0; g < G; g++) {
+            Volume* v = vs[g];
+            uint32_t* rk = v->ranks_.as<uint32_t>();
+            uint32_t* tmp = v->scan_tmp_.as<uint32_t>();
+            for (int L = 0; L < plan[g].D; L++) {
+                const BitDomain& d = plan[g].dom[L];
+                sa.push_back(ScanArgs{A(g, L), nullptr, 1, rk + plan[g].rk_off[L], d.nwords, tmp + plan[g].tmp_off[2 * L],
+                                      counts(g) + 2 * L});
+                if (plan[g].dilate)
+                    sa.push_back(ScanArgs{A(g, L), B(g, L), 2, rk + plan[g].rk_off[L] + d.nwords, d.nwords,
+                                          tmp + plan[g].tmp_off[2 * L + 1], counts(g) + 2 * L + 1});
+            }
+        }
+        XCHK(v0, launch_scan_multi(sa.data(), int(sa.size()), ex.ar, ex.s));
     }
-    XCHK(v0, launch_scan_multi(sa.data(), int(sa.size()), ex.ar, ex.s));
-    rc = drain(v0, ex, G);
+    rc = wait_host(v0, ex);
     if (rc) return rc;
 
     // per grid: pools sized from the counts, then nodes and links in one launch per kernel
-    std::vector<RootArgs> ra;
-    std::vector<FillArgs> cf;
     std::vector<EmitArgs> ea;
     std::vector<LinkArgs> la;
     for (int g = 0; g < G; g++) {
@@ -360,8 +424,6 @@ int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float
         r.root = v->pool_[0][D].dev.as<Node>();
         for (int a = 0; a < 3; a++) r.pos[a] = pl.rootPos[a];
         r.lev = D;
-        ra.push_back(r);
-        cf.push_back(FillArgs{v->pool_[1][D].dev.p, v->voxcnt(D), ID_UNDEF64, 1});
         // the brick table comes with the level-0 emission (one entry per box bit)
         u64* btab = nullptr;
         if (pl.dom[0].nbits <= BRICK_TAB_MAX) {
@@ -371,8 +433,11 @@ int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float
         }
         pl.btab = btab != nullptr;
         for (int L = 0; L < D; L++) {
-            ea.push_back(EmitArgs{LB[L], v->pool_[0][L].dev.as<Node>(), L > 0 ? 1 : 0, L == 0 ? btab : nullptr});
-            if (L > 0) cf.push_back(FillArgs{v->pool_[1][L].dev.p, v->pool_[1][L].lastEle * v->voxcnt(L), ID_UNDEF64, 1});
+            // level L's nodes and child lists; the root and its list with level 0
+            const int c = L > 0 ? L : D;
+            ea.push_back(EmitArgs{LB[L], v->pool_[0][L].dev.as<Node>(), L > 0 ? 1 : 0, L == 0 ? btab : nullptr,
+                                  v->pool_[1][c].dev.as<u64>(), v->pool_[1][c].lastEle * v->voxcnt(c),
+                                  L == 0 ? r : RootArgs{nullptr, {0, 0, 0}, 0}});
         }
         // gvdbLinkBricks walks from the top node; levels above it stay unlinked
         for (int L = 0; L < D; L++) {
@@ -382,8 +447,6 @@ int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float
                                   v->pool_[0][L].dev.as<Node>(), v->pool_[1][L + 1].dev.as<u64>(), v->voxcnt(L + 1)});
         }
     }
-    XCHK(v0, launch_write_root_multi(ra.data(), int(ra.size()), ex.ar, ex.s));
-    XCHK(v0, launch_fill_multi(cf.data(), int(cf.size()), ex.ar, ex.s));
     XCHK(v0, launch_emit_nodes_multi(ea.data(), int(ea.size()), ex.ar, ex.s));
     XCHK(v0, launch_link_level_multi(la.data(), int(la.size()), ex.ar, ex.s));
     for (int g = 0; g < G; g++) {
@@ -394,6 +457,7 @@ int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float
         v->dev_stale_ = false;
         v->topo_gen_++;
         v->btab_gen_ = plan[g].btab ? v->topo_gen_ : ~0u;
+        v->note_full_build(mnmx + 6 * g, odd[g] != 0, radius[g], plan[g].dom[0]);
     }
     return GVDB_OK;
 }
@@ -413,9 +477,9 @@ int Volume::accumulate_topology(int n, float radius, const float orig[3], int mi
     PointSrc P = pts_;
     P.n = n;
     XCHK(this, bbox_part_.ensure(size_t(BBOX_PART_WORDS) * 4));
-    BboxArgs ba{P, {orig[0], orig[1], orig[2]}, ex.dsmall + SM_BBOX, bbox_part_.as<uint32_t>()};
+    BboxArgs ba{P, {orig[0], orig[1], orig[2]}, ex.hsmall + SM_BBOX, bbox_part_.as<uint32_t>()};
     XCHK(this, launch_bbox_multi(&ba, 1, ex.ar, ex.s));
-    int rc = drain(this, ex, 1);
+    int rc = wait_host(this, ex);
     if (rc) return rc;
     float mnmx[6];
     for (int a = 0; a < 3; a++) {
@@ -621,7 +685,9 @@ int Volume::multi_finish_topology(Volume* const* vs, int G, bool commit, bool bo
             Volume* v = vs[g];
             Pool& p = v->pool_[0][0];
             float mnv[3] = {0, 0, 0}, mxv[3] = {0, 0, 0};
-            if (p.lastEle && v->dev_stale_) {
+            if (p.lastEle && v->all_leaves() && v->full_box_) {
+                for (int a = 0; a < 3; a++) { mnv[a] = v->full_min_[a]; mxv[a] = v->full_max_[a]; }
+            } else if (p.lastEle && v->dev_stale_) {
                 // host-built pools: bounds from the host mirror
                 Node* c = v->hnode(Elem(0, 0, 0));
                 for (int a = 0; a < 3; a++) mnv[a] = mxv[a] = float(c->mPos[a]);
@@ -687,6 +753,10 @@ int Volume::multi_update_atlas(Volume* const* vs, int G, const Exec& ex, int* fa
         }
         v->amap_max_ = u64(v->atlas_cnt_[0]) * v->atlas_cnt_[1] * v->atlas_cnt_[2];
         XCHK(v, v->amap_.ensure(size_t(v->amap_max_) * sizeof(AtlasNode)));
+        if (total && v->all_leaves() && total <= v->amap_max_) {
+            aa.push_back(AtlasArgs{v->make_tree(), nullptr, int(total), int(v->amap_max_)});
+            continue;
+        }
         fa.push_back(FillArgs{v->amap_.p, v->amap_max_ * 4, 0xFFFFFFFFull, 0});
         if (total) {
             XCHK(v, v->flags_.ensure(size_t(total) * 4));
@@ -696,7 +766,7 @@ int Volume::multi_update_atlas(Volume* const* vs, int G, const Exec& ex, int* fa
             fl.push_back(FlagArgs{t, v->flags_.as<uint32_t>(), int(total), 0});
             sa.push_back(ScanArgs{v->flags_.as<uint32_t>(), nullptr, 0, v->slot_scan_.as<uint32_t>(), total,
                                   v->scan_tmp_.as<uint32_t>(), nullptr});
-            aa.push_back(AtlasArgs{t, v->slot_scan_.as<uint32_t>(), int(total)});
+            aa.push_back(AtlasArgs{t, v->slot_scan_.as<uint32_t>(), int(total), 0});
         }
     }
     Volume* v0 = vs[0];
@@ -741,6 +811,7 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
         int sd, spb, R;
         u64 numSC, numMap;
         bool pull;
+        bool same;      // a full build: every leaf is linked, leaf i has subcell block i
         uint32_t linked = 0, total = 0, orphans = 0;
         PointSrc P;
         Tree t;
@@ -778,7 +849,10 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
                 FAILG(g, v->not_recordable("InsertPointsSubcell outside the bucketed path"));
             ex.cap->note(v);
         }
-        XCHK(v, v->sc_flags_.ensure(size_t(pl.numMap) * 4));
+        pl.same = v->all_leaves();
+        v->map_ready_ = !pl.same;
+        v->sc_map_n_ = int(pl.numMap);
+        if (!pl.same) XCHK(v, v->sc_flags_.ensure(size_t(pl.numMap) * 4));
         XCHK(v, v->sc_map_.ensure(size_t(pl.numMap) * 4));
         XCHK(v, v->sc_cnt_.ensure(size_t(pl.numSC) * 4));
         XCHK(v, v->sc_use_.ensure(size_t(pl.numSC) * 4));
@@ -804,6 +878,9 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
     // recorded before the last kernels, not after a wait for the stream
     const bool early = G == 1 && !ex.cap;
     auto small = [&](int g, int k) { return ex.dsmall + g * SMALL_WORDS + k; };
+    // words that kernels store and only the host reads: in host memory, except
+    // while recording (a graph copies them)
+    auto word = [&](int g, int k) { return (ex.cap ? ex.dsmall : ex.hsmall) + g * SMALL_WORDS + k; };
     auto tmp2 = [&](int g) { return vs[g]->scan_tmp_.as<uint32_t>() + scan_tmp_words(plan[g].numMap) + 64; };
     {
         std::vector<FlagArgs> fl;
@@ -813,22 +890,30 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
         for (int g = 0; g < G; g++) {
             Volume* v = vs[g];
             Plan& pl = plan[g];
-            fl.push_back(FlagArgs{pl.t, v->sc_flags_.as<uint32_t>(), int(pl.numMap), 1});
-            sa.push_back(ScanArgs{v->sc_flags_.as<uint32_t>(), nullptr, 0, v->sc_map_.as<uint32_t>(), pl.numMap,
-                                  v->scan_tmp_.as<uint32_t>(), small(g, SM_LINKED)});
-            fa.push_back(FillArgs{v->sc_cnt_.p, pl.numSC, 0, 0});
-            if (pl.pull) {
-                if (v->nbr_gen_ != v->topo_gen_) {
-                    // k_neighbors writes every brick's mask whole
-                    XCHK(v, v->nmask_.ensure(size_t(pl.numMap) * 4));
-                    XCHK(v, v->nbase_.ensure(size_t(pl.numMap) * 27 * 8));
-                    na.push_back(NbrArgs{pl.t, v->nbr_.as<int>(), int(pl.numMap), v->nmask_.as<uint32_t>(),
-                                         v->nbase_.as<long long>(), v->brick_tab()});
-                    v->nbr_gen_ = v->topo_gen_;
-                }
+            if (!pl.same) {
+                fl.push_back(FlagArgs{pl.t, v->sc_flags_.as<uint32_t>(), int(pl.numMap), 1});
+                sa.push_back(ScanArgs{v->sc_flags_.as<uint32_t>(), nullptr, 0, v->sc_map_.as<uint32_t>(), pl.numMap,
+                                      v->scan_tmp_.as<uint32_t>(), word(g, SM_LINKED)});
+            }
+            if (!pl.pull) {
+                fa.push_back(FillArgs{v->sc_cnt_.p, pl.numSC, 0, 0});
+                int rc = v->identity_map(ex.s);
+                if (rc) FAILG(g, rc);
+                continue;
+            }
+            XCHK(v, v->lenparts_.ensure(64 * 8));
+            if (v->nbr_gen_ != v->topo_gen_) {
+                // k_neighbors writes every brick's mask whole, and clears the
+                // counters of the bucketing
+                XCHK(v, v->nmask_.ensure(size_t(pl.numMap) * 4));
+                XCHK(v, v->nbase_.ensure(size_t(pl.numMap) * 27 * 8));
+                na.push_back(NbrArgs{pl.t, v->nbr_.as<int>(), int(pl.numMap), v->nmask_.as<uint32_t>(),
+                                     v->nbase_.as<long long>(), v->brick_tab(), v->bkt_cnt_.as<uint32_t>(), pl.spb,
+                                     v->lenparts_.as<u64>(), small(g, SM_ORPHANS)});
+                v->nbr_gen_ = v->topo_gen_;
+            } else {
                 fa.push_back(FillArgs{v->bkt_cnt_.p, pl.numMap * u64(pl.spb), 0, 0});
                 fa.push_back(FillArgs{small(g, SM_ORPHANS), 1, 0, 0});
-                XCHK(v, v->lenparts_.ensure(64 * 8));
                 fa.push_back(FillArgs{v->lenparts_.p, 64, 0, 1});
             }
         }
@@ -841,8 +926,7 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
         std::vector<BucketArgs> ba;
         std::vector<ScanArgs> sb, sc;
         std::vector<ScatterArgs> sca;
-        std::vector<const u64*> lp;
-        std::vector<u64*> lo;
+        std::vector<SumArgs> sums;
         for (int g = 0; g < G; g++) {
             Volume* v = vs[g];
             Plan& pl = plan[g];
@@ -853,6 +937,7 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
                                              v->sc_cnt_.as<uint32_t>(), rule, ex.s));
                 XCHK(v, launch_sum_u32(v->sc_cnt_.as<uint32_t>(), pl.numSC, reinterpret_cast<u64*>(small(g, SM_LEN)),
                                        ex.s));
+                XCHK(v, hipMemcpyAsync(word(g, SM_LEN), small(g, SM_LEN), 8, hipMemcpyDeviceToHost, ex.s));
                 sc.push_back(ScanArgs{v->sc_cnt_.as<uint32_t>(), nullptr, 0, v->sc_off_.as<uint32_t>(), pl.numSC,
                                       tmp2(g), small(g, SM_TOTAL)});
                 continue;
@@ -861,8 +946,8 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
             ba.push_back(BucketArgs{pl.t, pl.P, scs, pl.spb, {tr[0], tr[1], tr[2]}, v->bkt_key_.as<uint32_t>(),
                                     v->bkt_slot_.as<uint32_t>(), v->bkt_cnt_.as<uint32_t>(), small(g, SM_ORPHANS),
                                     v->nmask_.as<uint32_t>(), radius[g], v->lenparts_.as<u64>(), rule, v->brick_tab()});
-            lp.push_back(v->lenparts_.as<u64>());
-            lo.push_back(reinterpret_cast<u64*>(small(g, SM_LEN)));
+            sums.push_back(SumArgs{v->lenparts_.as<u64>(), reinterpret_cast<u64*>(word(g, SM_LEN)),
+                                   small(g, SM_ORPHANS), ex.cap ? nullptr : word(g, SM_ORPHANS)});
             sb.push_back(ScanArgs{v->bkt_cnt_.as<uint32_t>(), nullptr, 0, v->bkt_off_.as<uint32_t>(), nb, tmp2(g),
                                   small(g, SM_BUCKETS)});
             // SetPoints' colours travel with the bucketed points (fourth word)
@@ -873,14 +958,11 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
             v->bkt_clr_ = clr;
         }
         XCHK(v0, launch_bucket_points_multi(ba.data(), int(ba.size()), ex.ar, ex.s));
-        XCHK(v0, launch_sum_parts_multi(lp.data(), lo.data(), int(lp.size()), ex.ar, ex.s));
-        if (early) {
-            // every word the host reads below is final here: it comes back
-            // while the bucket scan and scatter still run, and the gather the
-            // caller launches next queues behind them
-            XCHK(v0, hipMemcpyAsync(ex.hsmall, ex.dsmall, SMALL_WORDS * 4, hipMemcpyDeviceToHost, ex.s));
-            XCHK(v0, hipEventRecord(v0->small_ev_, ex.s));
-        }
+        XCHK(v0, launch_sum_parts_multi(sums.data(), int(sums.size()), ex.ar, ex.s));
+        // every word the host reads below is final here: the host returns while
+        // the bucket scan and scatter still run, and the gather the caller
+        // launches next queues behind them
+        if (early) XCHK(v0, hipEventRecord(v0->small_ev_, ex.s));
         XCHK(v0, launch_scan_multi(sb.data(), int(sb.size()), ex.ar, ex.s));
         XCHK(v0, launch_bucket_scatter_multi(sca.data(), int(sca.size()), ex.ar, ex.s));
         XCHK(v0, launch_scan_multi(sc.data(), int(sc.size()), ex.ar, ex.s));
@@ -889,7 +971,7 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
     if (early)
         XCHK(v0, hipEventSynchronize(v0->small_ev_));
     else
-        rc = drain(v0, ex, G);
+        rc = ex.cap ? drain(v0, ex, G) : wait_host(v0, ex);
     if (rc) return rc;
     if (ex.cap) {
         // recording: the entry counts arrive with the replay (graph_synchronize
@@ -917,7 +999,7 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
     bool redo = false;
     for (int g = 0; g < G; g++) {
         Plan& pl = plan[g];
-        pl.linked = ex.hsmall[g * SMALL_WORDS + SM_LINKED];
+        pl.linked = pl.same ? uint32_t(pl.numMap) : ex.hsmall[g * SMALL_WORDS + SM_LINKED];
         pl.orphans = pl.pull ? ex.hsmall[g * SMALL_WORDS + SM_ORPHANS] : 0;
         {
             // the exact entry total in 64 bits (the u32 scan's wraps)
@@ -929,6 +1011,8 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
             Volume* v = vs[g];
             pl.pull = false;
             redo = true;
+            rc = v->identity_map(ex.s);
+            if (rc) FAILG(g, rc);
             XCHK(v, launch_fill_u32(v->sc_cnt_.as<uint32_t>(), 0u, pl.numSC, ex.s));
             XCHK(v, launch_count_subcell(pl.t, pl.P, scs, pl.spb, trans3 + 3 * g, radius[g], v->sc_map_.as<uint32_t>(),
                                          v->sc_cnt_.as<uint32_t>(), rule, ex.s));
@@ -936,10 +1020,11 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
                                    ex.s));
             XCHK(v, launch_scan_u32(v->sc_cnt_.as<uint32_t>(), nullptr, 0, v->sc_off_.as<uint32_t>(), pl.numSC,
                                     small(g, SM_TOTAL), tmp2(g), ex.s));
+            XCHK(v, hipMemcpyAsync(word(g, SM_LEN), small(g, SM_LEN), 8, hipMemcpyDeviceToHost, ex.s));
         }
     }
     if (redo) {
-        rc = drain(v0, ex, G);
+        rc = wait_host(v0, ex);
         if (rc) return rc;
         for (int g = 0; g < G; g++)
             if (!plan[g].pull) {
@@ -1010,6 +1095,10 @@ int Volume::multi_materialize(Volume* const* vs, int G, const Exec& ex, int* fai
         XCHK(v, v->sc_pos_.ensure(size_t(numSC) * 12));
         XCHK(v, v->sc_nid_.ensure(size_t(numSC) * 4));
         XCHK(v, v->scan_tmp_.ensure(scan_tmp_words(numSC) * 4 + 256));
+        {
+            const int rc = v->identity_map(ex.s);
+            if (rc) FAILG(g, rc);
+        }
         Tree t = v->make_tree();
         fa.push_back(FillArgs{v->sc_cnt_.p, numSC, 0, 0});
         PullArgs a{t, int(numMap), scs, v->bkt_R_, v->bkt_radius_, v->nbr_.as<int>(), v->bkt_cnt_.as<uint32_t>(),

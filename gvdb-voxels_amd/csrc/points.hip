@@ -1,5 +1,6 @@
 // points.hip -- atlas slot assignment, subcell binning and the density gather.
 #include "kernels.h"
+#include <algorithm>
 #include <type_traits>
 #include "tree_device.h"
 #include <hip/hip_fp16.h>
@@ -18,10 +19,13 @@ __device__ inline void k_update_atlas_body(const AtlasArgs& a, uint32_t bid, uin
     const Tree& t = a.t;
     const uint32_t* slot_scan = a.slot_scan;
     int i = bid * 256 + threadIdx.x;
-    if (i >= a.n) return;
+    if (i >= a.n) {
+        if (i < a.map_n) t.amap[i] = AtlasNode{{-1, -1, -1}, -1};
+        return;
+    }
     Node* n = t.nodes[0] + i;
-    if (!n->mFlags) return;
-    u64 id = slot_scan[i];
+    if (slot_scan && !n->mFlags) return;
+    u64 id = slot_scan ? u64(slot_scan[i]) : u64(i);
     u64 a2 = u64(t.atlas_cnt[0]) * t.atlas_cnt[1];
     int pz = int(id / a2);
     id -= u64(pz) * a2;
@@ -54,7 +58,7 @@ static hipError_t launch_per_item(const A* a, const uint32_t* items, int G, Aren
 
 hipError_t launch_update_atlas_multi(const AtlasArgs* a, int G, Arena* ar, hipStream_t s) {
     std::vector<uint32_t> items(G);
-    for (int g = 0; g < G; g++) items[g] = uint32_t(a[g].n);
+    for (int g = 0; g < G; g++) items[g] = uint32_t(std::max(a[g].n, a[g].map_n));
     return launch_per_item<AtlasArgs, k_update_atlas>(a, items.data(), G, ar, s, 256);
 }
 
@@ -670,24 +674,23 @@ __device__ inline void k_bucket_points_body(const BucketArgs& a, uint32_t bid, u
 }
 
 // Sum of a grid's LEN_PARTS entry counters into its result word.
-struct SumArgs {
-    const u64* parts;
-    u64* out;
-};
+// (and the orphan count beside it: both go to host memory when the host is the
+// only reader)
 __device__ inline void k_sum_parts_body(const SumArgs& a, uint32_t, uint32_t) {
     u64 v = threadIdx.x < LEN_PARTS ? a.parts[threadIdx.x] : 0ull;
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
-    if (threadIdx.x == 0) *a.out = v;
+    if (threadIdx.x == 0) {
+        store_word(a.out, v);
+        if (a.orphans_out) store_word(a.orphans_out, *a.orphans);
+    }
 }
 GVDB_MULTI(k_sum_parts, SumArgs, 64)
 
-hipError_t launch_sum_parts_multi(const u64* const* parts, u64* const* out, int G, Arena* ar, hipStream_t s) {
-    std::vector<SumArgs> a(G);
+hipError_t launch_sum_parts_multi(const SumArgs* a, int G, Arena* ar, hipStream_t s) {
     std::vector<uint32_t> nb(G, 1u);
-    for (int g = 0; g < G; g++) a[g] = SumArgs{parts[g], out[g]};
     MultiLaunch L;
-    hipError_t e = multi_setup(ar, a.data(), nb.data(), G, s, L);
+    hipError_t e = multi_setup(ar, a, nb.data(), G, s, L);
     if (e != hipSuccess || L.blocks == 0) return e;
     hipLaunchKernelGGL(k_sum_parts, dim3(L.blocks), dim3(64), 0, s, a[0], L.map);
     return hipGetLastError();

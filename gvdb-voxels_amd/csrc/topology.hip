@@ -18,6 +18,7 @@
 // same set because power-of-two node ranges nest.
 #include "kernels.h"
 #include "tree_device.h"
+#include <algorithm>
 
 namespace gvdb {
 
@@ -40,6 +41,7 @@ static uint32_t grid_for(u64 items, uint32_t cap) {
 // GetBoundingBox's split + Thrust min/max (src/gvdb_volume_gvdb.cpp:5404-5467).
 __device__ inline void k_bbox_body(const BboxArgs& a, uint32_t bid, uint32_t nblk) {
     float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+    float odd = 0.0f;     // becomes a NaN with a coordinate that is none or infinite
     const PointSrc& P = a.pts;
     if (P.stride == 12 && P.off == 0 && P.n < (1 << 30) && (reinterpret_cast<uintptr_t>(P.base) & 15) == 0) {
         // packed float3: four points = three float4 per thread (axes fixed:
@@ -47,9 +49,9 @@ __device__ inline void k_bbox_body(const BboxArgs& a, uint32_t bid, uint32_t nbl
         const float4* v = reinterpret_cast<const float4*>(P.base);
         const uint32_t ng = uint32_t(P.n) / 4u;
         const float ox = a.o[0], oy = a.o[1], oz = a.o[2];
-        auto ux = [&](float f) { f += ox; mn[0] = fminf(mn[0], f); mx[0] = fmaxf(mx[0], f); };
-        auto uy = [&](float f) { f += oy; mn[1] = fminf(mn[1], f); mx[1] = fmaxf(mx[1], f); };
-        auto uz = [&](float f) { f += oz; mn[2] = fminf(mn[2], f); mx[2] = fmaxf(mx[2], f); };
+        auto ux = [&](float f) { f += ox; odd = __builtin_fmaf(f, 0.0f, odd); mn[0] = fminf(mn[0], f); mx[0] = fmaxf(mx[0], f); };
+        auto uy = [&](float f) { f += oy; odd = __builtin_fmaf(f, 0.0f, odd); mn[1] = fminf(mn[1], f); mx[1] = fmaxf(mx[1], f); };
+        auto uz = [&](float f) { f += oz; odd = __builtin_fmaf(f, 0.0f, odd); mn[2] = fminf(mn[2], f); mx[2] = fmaxf(mx[2], f); };
         for (uint32_t g = bid * 256 + threadIdx.x; g < ng; g += nblk * 256) {
             const float4 q0 = v[3 * u64(g)], q1 = v[3 * u64(g) + 1], q2 = v[3 * u64(g) + 2];
             ux(q0.x); uy(q0.y); uz(q0.z); ux(q0.w);
@@ -65,7 +67,11 @@ __device__ inline void k_bbox_body(const BboxArgs& a, uint32_t bid, uint32_t nbl
             const float* p = point_at(P, i);
             float w[3] = {p[0] + a.o[0], p[1] + a.o[1], p[2] + a.o[2]};
 #pragma unroll
-            for (int k = 0; k < 3; k++) { mn[k] = fminf(mn[k], w[k]); mx[k] = fmaxf(mx[k], w[k]); }
+            for (int k = 0; k < 3; k++) {
+                mn[k] = fminf(mn[k], w[k]);
+                mx[k] = fmaxf(mx[k], w[k]);
+                odd = __builtin_fmaf(w[k], 0.0f, odd);
+            }
         }
     }
 #pragma unroll
@@ -77,50 +83,53 @@ __device__ inline void k_bbox_body(const BboxArgs& a, uint32_t bid, uint32_t nbl
         }
     }
     __shared__ float smn[4][3], smx[4][3];
+    __shared__ uint32_t sodd[4];
     int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0)
+    const bool any_odd = __any(odd != odd);
+    if ((threadIdx.x & 63) == 0) {
         for (int k = 0; k < 3; k++) { smn[wave][k] = mn[k]; smx[wave][k] = mx[k]; }
+        sodd[wave] = any_odd ? 1u : 0u;
+    }
     __syncthreads();
-    // each block stores its six keys; k_bbox_reduce combines them (a kernel
+    // each block stores its six keys and whether it met an odd coordinate; k_bbox_reduce combines them (a kernel
     // boundary orders the stores: no same-address atomics, no fences)
     if (threadIdx.x < 3) {
         int k = threadIdx.x;
         float m0 = smn[0][k], m1 = smx[0][k];
         for (int w = 1; w < 4; w++) { m0 = fminf(m0, smn[w][k]); m1 = fmaxf(m1, smx[w][k]); }
-        a.part[bid * 6 + k] = float_key(m0);
-        a.part[bid * 6 + 3 + k] = float_key(m1);
+        a.part[bid * 7 + k] = float_key(m0);
+        a.part[bid * 7 + 3 + k] = float_key(m1);
+        if (k == 0) a.part[bid * 7 + 6] = sodd[0] | sodd[1] | sodd[2] | sodd[3];
     }
 }
 GVDB_MULTI(k_bbox, BboxArgs, 256)
 
-// One block per grid: the minimum and maximum over the blocks' keys.
+// One block per grid: the minimum and maximum over the blocks' keys (word 6:
+// any of them set).
 __device__ inline void k_bbox_reduce_body(const BboxArgs& a, uint32_t, uint32_t) {
-    uint32_t k6[6] = {~0u, ~0u, ~0u, 0u, 0u, 0u};
+    uint32_t k7[7] = {~0u, ~0u, ~0u, 0u, 0u, 0u, 0u};
     for (uint32_t j = threadIdx.x; j < a.nparts; j += 256) {
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-            k6[k] = min(k6[k], a.part[j * 6 + k]);
-            k6[3 + k] = max(k6[3 + k], a.part[j * 6 + 3 + k]);
-        }
+        for (int k = 0; k < 7; k++) k7[k] = k < 3 ? min(k7[k], a.part[j * 7 + k]) : max(k7[k], a.part[j * 7 + k]);
     }
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
+    for (int k = 0; k < 7; k++) {
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) {
-            k6[k] = min(k6[k], uint32_t(__shfl_xor(int(k6[k]), d, 64)));
-            k6[3 + k] = max(k6[3 + k], uint32_t(__shfl_xor(int(k6[3 + k]), d, 64)));
+            const uint32_t o = uint32_t(__shfl_xor(int(k7[k]), d, 64));
+            k7[k] = k < 3 ? min(k7[k], o) : max(k7[k], o);
         }
     }
-    __shared__ uint32_t sk[4][6];
+    __shared__ uint32_t sk[4][7];
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0)
-        for (int k = 0; k < 6; k++) sk[wave][k] = k6[k];
+        for (int k = 0; k < 7; k++) sk[wave][k] = k7[k];
     __syncthreads();
-    if (threadIdx.x < 6) {
+    if (threadIdx.x < 7) {
         const int k = threadIdx.x;
         uint32_t m = sk[0][k];
         for (int w = 1; w < 4; w++) m = k < 3 ? min(m, sk[w][k]) : max(m, sk[w][k]);
-        a.keys6[k] = m;
+        store_word(a.keys7 + k, m);
     }
 }
 GVDB_MULTI(k_bbox_reduce, BboxArgs, 256)
@@ -293,15 +302,15 @@ __device__ inline void k_pack_bytes_body(const MarkArgs& a, uint32_t bid, uint32
 }
 GVDB_MULTI(k_pack_bytes, MarkArgs, 256)
 
-hipError_t launch_mark_points_multi(const MarkArgs* a, int G, Arena* ar, hipStream_t s) {
+hipError_t launch_mark_points_multi(const MarkArgs* a, int G, Arena* ar, hipStream_t s, bool pack) {
     std::vector<uint32_t> nb(G), nb2(G), nb3(G);
     bool any_mask = false, any_bytes = false;
     for (int g = 0; g < G; g++) {
         nb[g] = a[g].pts.n > 0 ? grid_for(u64(a[g].pts.n), 16384) : 0;
         nb2[g] = a[g].masks && !a[g].bytes ? grid_for(a[g].d0.nbits, 16384) : 0;
-        nb3[g] = a[g].bytes ? grid_for(a[g].d0.nwords, 16384) : 0;
+        nb3[g] = pack && a[g].bytes ? grid_for(a[g].d0.nwords, 16384) : 0;
         any_mask |= a[g].masks != nullptr && !a[g].bytes;
-        any_bytes |= a[g].bytes != nullptr;
+        any_bytes |= pack && a[g].bytes != nullptr;
     }
     MultiLaunch L;
     hipError_t e = multi_setup(ar, a, nb.data(), G, s, L);
@@ -387,6 +396,112 @@ hipError_t launch_mark_parents_multi(const ParentArgs* a, int G, Arena* ar, hipS
     return hipGetLastError();
 }
 
+// The byte marks of a small box to bitmaps, parents and ranks of every level in
+// one workgroup per grid, the bitmaps in LDS: what k_pack_bytes, k_mark_parents
+// and the scans do in seven launches or more, each a few microseconds of a few
+// CUs' work.  Bound by its own latency: the bytes come in four groups of loads
+// in flight, parents are found a row of children per thread.
+__global__ __launch_bounds__(1024) void k_box_levels(const BoxArgs* recs, BoxArgs one) {
+    const BoxArgs& a = recs ? recs[blockIdx.x] : one;
+    __shared__ uint32_t bm[BOX_WORDS];
+    __shared__ uint32_t wsum[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int sets = a.dilate ? 2 : 1;
+    // level 0
+    const uint32_t n0 = uint32_t(a.dom[0].nwords);
+    for (uint32_t w0 = uint32_t(tid); w0 < n0 * uint32_t(sets); w0 += 4096) {
+        uint32_t m[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t w = w0 + uint32_t(k) * 1024u;
+            m[k] = w < n0 * uint32_t(sets) ? pack32(a.bytes + u64(w) * 32) : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t w = w0 + uint32_t(k) * 1024u;
+            if (w < n0 * uint32_t(sets)) bm[w] = m[k];
+        }
+    }
+    uint32_t at = n0 * uint32_t(sets);
+    for (int L = 1; L < a.D; L++) at += uint32_t(a.dom[L].nwords) * uint32_t(sets);
+    for (uint32_t w = n0 * uint32_t(sets) + uint32_t(tid); w < at; w += 1024) bm[w] = 0;
+    __syncthreads();
+    // parents: a thread per row (x, y) of children, whose runs of 2^shift z
+    // bits each have one parent
+    uint32_t co = 0, po = n0 * uint32_t(sets);
+    for (int L = 1; L < a.D; L++) {
+        const BitDomain &c = a.dom[L - 1], &p = a.dom[L];
+        const uint32_t cw = uint32_t(c.nwords), pw = uint32_t(p.nwords);
+        const int s = a.logdim[L];
+        const uint32_t dy = uint32_t(c.dim[1]), dz = uint32_t(c.dim[2]), rows = uint32_t(c.dim[0]) * dy;
+        for (uint32_t r = uint32_t(tid); r < rows; r += 1024) {
+            const uint32_t x = r / dy, y = r - x * dy;
+            const uint32_t prow = (uint32_t(((int(x) + c.lo[0]) >> s) - p.lo[0]) * uint32_t(p.dim[1]) +
+                                   uint32_t(((int(y) + c.lo[1]) >> s) - p.lo[1])) * uint32_t(p.dim[2]);
+            for (int pz = 0; pz < p.dim[2]; pz++) {
+                const int z0 = max((pz + p.lo[2]) << s, c.lo[2]) - c.lo[2],
+                          z1 = min((((pz + p.lo[2]) + 1) << s) - 1, c.lo[2] + int(dz) - 1) - c.lo[2];
+                if (z0 > z1) continue;
+                const uint32_t i0 = r * dz + uint32_t(z0), i1 = r * dz + uint32_t(z1), b = prow + uint32_t(pz);
+                if (any_bits(bm + co, i0, i1)) atomicOr(&bm[po + (b >> 5)], 1u << (b & 31));
+                if (sets == 2 && any_bits(bm + co + cw, i0, i1)) atomicOr(&bm[po + pw + (b >> 5)], 1u << (b & 31));
+            }
+        }
+        __syncthreads();
+        co = po;
+        po += pw * uint32_t(sets);
+    }
+    // bitmaps out, ranks by exclusive scans of the popcounts, 1024 words a step
+    uint32_t off = 0;
+    for (int L = 0; L < a.D; L++) {
+        const uint32_t nw = uint32_t(a.dom[L].nwords);
+        for (int k = 0; k < sets; k++) {
+            uint32_t base = 0;
+            for (uint32_t w0 = 0; w0 < nw; w0 += 1024) {
+                const uint32_t w = w0 + uint32_t(tid);
+                uint32_t v = 0;
+                if (w < nw) {
+                    const uint32_t av = bm[off + w], x = k == 0 ? av : bm[off + nw + w];
+                    a.bitmaps[off + uint32_t(k) * nw + w] = x;
+                    v = uint32_t(__popc(k == 0 ? av : x & ~av));
+                }
+                uint32_t x = v;
+#pragma unroll
+                for (int d = 1; d < 64; d <<= 1) {
+                    const uint32_t y = __shfl_up(x, d, 64);
+                    if (lane >= d) x += y;
+                }
+                __syncthreads();
+                if (lane == 63) wsum[wave] = x;
+                __syncthreads();
+                uint32_t pre = base, tot = 0;
+#pragma unroll
+                for (int q = 0; q < 16; q++) {
+                    if (q < wave) pre += wsum[q];
+                    tot += wsum[q];
+                }
+                if (w < nw) a.ranks[off + uint32_t(k) * nw + w] = pre + x - v;
+                base += tot;
+            }
+            if (tid == 0) store_word(a.counts + 2 * L + k, base);
+        }
+        off += nw * uint32_t(sets);
+    }
+}
+
+hipError_t launch_box_levels_multi(const BoxArgs* a, int G, Arena* ar, hipStream_t s) {
+    if (G <= 0) return hipSuccess;
+    const BoxArgs* recs = nullptr;
+    if (G > 1) {
+        hipError_t e = hipSuccess;
+        if (!ar) return hipErrorInvalidValue;
+        recs = static_cast<const BoxArgs*>(ar->push(a, sizeof(BoxArgs) * size_t(G), s, e));
+        if (!recs) return e;
+    }
+    hipLaunchKernelGGL(k_box_levels, dim3(unsigned(G)), dim3(1024), 0, s, recs, a[0]);
+    return hipGetLastError();
+}
+
 __device__ inline void write_node(Node* n, int lev, int x, int y, int z, int range, u64 clist) {
     Node v;
     v.mLev = uint8_t(lev);
@@ -402,10 +517,30 @@ __device__ inline void write_node(Node* n, int lev, int x, int y, int z, int ran
     *n = v;
 }
 
+// Root node (SetupNode at the top level, src/gvdb_volume_gvdb.cpp:1289-1300).
+__device__ inline void write_root(const RootArgs& a) {
+    Node v;
+    v.mLev = uint8_t(a.lev);
+    v.mFlags = 1;
+    v.mPriority = 0;
+    v.pad = 0;
+    v.mPos[0] = a.pos[0]; v.mPos[1] = a.pos[1]; v.mPos[2] = a.pos[2];
+    v.mValue[0] = v.mValue[1] = v.mValue[2] = -1;
+    v.mVRange[0] = v.mVRange[1] = v.mVRange[2] = 0.f;
+    v.mParent = ID_UNDEFL;
+    v.mChildList = Elem(1, a.lev, 0);
+    v.mMask = 0;
+    *a.root = v;
+}
+
 // Node creation in sorted key order (src/gvdb_volume_gvdb.cpp:1308-1331 for the
 // first pass, :965-988 for the appended dilation nodes).
+// The same launch empties the level's child lists and, on level 0, writes the
+// root and empties its list (linking comes in the next launch).
 __device__ inline void k_emit_nodes_body(const EmitArgs& a, uint32_t bid, uint32_t nblk) {
     const LevelBuild& L = a.L;
+    for (u64 i = u64(bid) * 256 + threadIdx.x; i < a.fill_n; i += u64(nblk) * 256) a.fill[i] = ID_UNDEF64;
+    if (a.root.root && bid == 0 && threadIdx.x == 0) write_root(a.root);
     if (L.dom.nbits <= PER_BIT_MAX) {
         const bool dil = L.bmB != L.bmA && L.bmB;
         for (u64 i = u64(bid) * 256 + threadIdx.x; i < L.dom.nbits; i += u64(nblk) * 256) {
@@ -458,7 +593,7 @@ GVDB_MULTI(k_emit_nodes, EmitArgs, 256)
 hipError_t launch_emit_nodes_multi(const EmitArgs* a, int G, Arena* ar, hipStream_t s) {
     std::vector<uint32_t> nb(G);
     for (int g = 0; g < G; g++)
-        nb[g] = grid_for(a[g].L.dom.nbits <= PER_BIT_MAX ? a[g].L.dom.nbits : a[g].L.dom.nwords, 16384);
+        nb[g] = grid_for(std::max(a[g].L.dom.nbits <= PER_BIT_MAX ? a[g].L.dom.nbits : a[g].L.dom.nwords, a[g].fill_n), 16384);
     MultiLaunch L;
     hipError_t e = multi_setup(ar, a, nb.data(), G, s, L);
     if (e != hipSuccess || L.blocks == 0) return e;
@@ -514,21 +649,8 @@ hipError_t launch_link_level_multi(const LinkArgs* a, int G, Arena* ar, hipStrea
     return hipGetLastError();
 }
 
-// Root node (SetupNode at the top level, src/gvdb_volume_gvdb.cpp:1289-1300).
 __device__ inline void k_write_root_body(const RootArgs& a, uint32_t, uint32_t) {
-    if (threadIdx.x != 0) return;
-    Node v;
-    v.mLev = uint8_t(a.lev);
-    v.mFlags = 1;
-    v.mPriority = 0;
-    v.pad = 0;
-    v.mPos[0] = a.pos[0]; v.mPos[1] = a.pos[1]; v.mPos[2] = a.pos[2];
-    v.mValue[0] = v.mValue[1] = v.mValue[2] = -1;
-    v.mVRange[0] = v.mVRange[1] = v.mVRange[2] = 0.f;
-    v.mParent = ID_UNDEFL;
-    v.mChildList = Elem(1, a.lev, 0);
-    v.mMask = 0;
-    *a.root = v;
+    if (threadIdx.x == 0) write_root(a);
 }
 GVDB_MULTI(k_write_root, RootArgs, 64)
 

@@ -71,11 +71,14 @@ hipError_t multi_setup_raw(Arena* ar, const void* args, size_t rec, const uint32
     }
     if (!ar) return hipErrorInvalidValue;
     hipError_t e = hipSuccess;
-    void* t = ar->push(args, rec * size_t(G), s, e);
+    // one copy: the records, then first[]
+    const size_t nrec = (rec * size_t(G) + 15) & ~size_t(15);
+    std::vector<unsigned char> both(nrec + first.size() * 4);
+    memcpy(both.data(), args, rec * size_t(G));
+    memcpy(both.data() + nrec, first.data(), first.size() * 4);
+    unsigned char* t = static_cast<unsigned char*>(ar->push(both.data(), both.size(), s, e));
     if (!t) return e;
-    void* f = ar->push(first.data(), first.size() * 4, s, e);
-    if (!f) return e;
-    out.map = MultiMap{G, reinterpret_cast<const uint32_t*>(f), t};
+    out.map = MultiMap{G, reinterpret_cast<const uint32_t*>(t + nrec), t};
     return hipSuccess;
 }
 
@@ -122,6 +125,17 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t v, u64 n, hipStream_t s) {
 hipError_t launch_fill_u64(u64* p, u64 v, u64 n, hipStream_t s) {
     FillArgs a{p, n, v, 1};
     return n ? launch_fill_multi(&a, 1, nullptr, s) : hipSuccess;
+}
+
+__global__ __launch_bounds__(256) void k_iota(uint32_t* out, u64 n) {
+    const u64 i = u64(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n) out[i] = uint32_t(i);
+}
+
+hipError_t launch_iota(uint32_t* out, u64 n, hipStream_t s) {
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_iota, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, out, n);
+    return hipGetLastError();
 }
 
 // ------------------------------------------------------------ 64-bit sum
@@ -194,18 +208,37 @@ __device__ inline void k_scan_tile_body(const ScanArgs& a, uint32_t bid, uint32_
     }
     if (threadIdx.x == 0) {
         a.sums[bid] = tile;
-        if (a.total && nblk == 1) *a.total = tile;
+        if (a.total && nblk == 1) store_word(a.total, tile);
     }
 }
 GVDB_MULTI(k_scan_tile, ScanArgs, SCAN_THREADS)
 
+// Adds the sum of the tiles before a tile to it.  `scanned`: offs[] holds those
+// sums; otherwise the tiles' own sums, which each block adds up itself (up to
+// SCAN_DIRECT of them, 16 loads a thread: a launch fewer than scanning them
+// first), and the last block stores the total.
+static const uint32_t SCAN_DIRECT = 4096;
 struct AddArgs {
     uint32_t* out;
     u64 n;
     const uint32_t* offs;
+    int scanned;
+    uint32_t* total;
 };
-__device__ inline void k_scan_add_body(const AddArgs& a, uint32_t bid, uint32_t) {
-    uint32_t add = a.offs[bid];
+__device__ inline void k_scan_add_body(const AddArgs& a, uint32_t bid, uint32_t nblk) {
+    uint32_t add = 0;
+    if (a.scanned) {
+        add = a.offs[bid];
+    } else {
+        __shared__ uint32_t part[SCAN_THREADS / 64];
+        for (uint32_t j = threadIdx.x; j < bid; j += SCAN_THREADS) add += a.offs[j];
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) add += __shfl_xor(add, d, 64);
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = add;
+        __syncthreads();
+        add = part[0] + part[1] + part[2] + part[3];
+        if (a.total && bid == nblk - 1 && threadIdx.x == 0) store_word(a.total, add + a.offs[bid]);
+    }
     u64 base = u64(bid) * SCAN_TILE;
 #pragma unroll
     for (int k = 0; k < SCAN_PER_THREAD; k++) {
@@ -244,17 +277,19 @@ hipError_t launch_scan_multi(const ScanArgs* a, int G, Arena* ar, hipStream_t s)
     hipLaunchKernelGGL(k_scan_tile, dim3(L.blocks), dim3(SCAN_THREADS), 0, s, a[0], L.map);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    // segments of more than one tile: scan their tile sums in place, add back
+    // segments of more than one tile: their tile sums (scanned in place when
+    // there are many) added back
     std::vector<ScanArgs> up;
     std::vector<AddArgs> add;
     std::vector<uint32_t> addnb;
     for (int g = 0; g < G; g++) {
         if (nb[g] <= 1) continue;
-        up.push_back(ScanArgs{a[g].sums, nullptr, 0, a[g].sums, nb[g], a[g].sums + nb[g] + 1, a[g].total});
-        add.push_back(AddArgs{a[g].out, a[g].n, a[g].sums});
+        const bool direct = nb[g] <= SCAN_DIRECT;
+        if (!direct) up.push_back(ScanArgs{a[g].sums, nullptr, 0, a[g].sums, nb[g], a[g].sums + nb[g] + 1, a[g].total});
+        add.push_back(AddArgs{a[g].out, a[g].n, a[g].sums, direct ? 0 : 1, a[g].total});
         addnb.push_back(nb[g]);
     }
-    if (up.empty()) return hipSuccess;
+    if (add.empty()) return hipSuccess;
     e = launch_scan_multi(up.data(), int(up.size()), ar, s);
     if (e != hipSuccess) return e;
     MultiLaunch L2;

@@ -71,7 +71,7 @@ int Volume::finish_recorded_insert(const uint32_t* slot) {
     memcpy(&total, slot + SM_LEN, 8);
     if (total > 0x7FFFFFFFull) return fail(GVDB_ERR_RANGE, "graph replay: more than 2^31 subcell entries");
     sc_len_ = int(total);
-    sc_bricks_ = int(slot[SM_LINKED]);
+    sc_bricks_ = all_leaves() ? sc_map_n_ : int(slot[SM_LINKED]);
     return GVDB_OK;
 }
 
@@ -935,6 +935,14 @@ int Volume::read_atlas_map(void* dst) {
     return GVDB_OK;
 }
 
+int Volume::identity_map(hipStream_t s) {
+    if (map_ready_ || sc_map_n_ <= 0) return GVDB_OK;
+    HIPCHK(sc_map_.ensure(size_t(sc_map_n_) * 4));
+    HIPCHK(launch_iota(sc_map_.as<uint32_t>(), u64(sc_map_n_), s));
+    map_ready_ = true;
+    return GVDB_OK;
+}
+
 int Volume::read_subcells(int which, void* dst, u64* count) {
     if (entries_stale_ && dst) {
         Volume* v = this;
@@ -949,7 +957,12 @@ int Volume::read_subcells(int which, void* dst, u64* count) {
         case 2: b = &sc_pos_; n = num_sc_; esz = 12; break;
         case 3: b = &sc_nid_; n = num_sc_; break;
         case 4: b = &sc_pnt_; n = sc_len_; esz = 12; break;
-        case 5: b = &sc_map_; n = sc_map_n_; break;
+        case 5:
+            if (dst) {
+                const int rc = identity_map(stream);
+                if (rc) return rc;
+            }
+            b = &sc_map_; n = sc_map_n_; break;
         case 6:
             if (!sc16_valid_) return fail(GVDB_ERR_STATE, "read_subcells: no InsertPointsSubcell_FP16 entries");
             b = &sc_pnt16_; n = sc_len_; esz = 6; break;

@@ -194,7 +194,8 @@ public:
     static int multi_rebuild_topology(Volume* const* v, int G, const int* n, const float* radius, const float* orig3,
                                       const Exec& ex, int* failed);
     static int multi_full_build(Volume* const* v, int G, const int* n, const float* radius, const float* orig3,
-                                const int* depth, const int* rootPos, const float* mnmx, const Exec& ex, int* failed);
+                                const int* depth, const int* rootPos, const float* mnmx, const uint8_t* odd, const Exec& ex,
+                                int* failed);
     int incremental_topology(int n, float radius, const float orig[3], int D, bool accum, const float* mnmx,
                              const Exec& ex);
     // the per-level brick boxes of a full build (false: level-0 coordinates
@@ -216,6 +217,7 @@ public:
     // chanC >= 0: also the colour channel, from the colours the insert carried
     static int multi_gather(Volume* const* v, int G, int scs, const int* len, const float* radius, int chanD, bool accum,
                             bool levelset, const Exec& ex, int* failed, bool fp16 = false, int chanC = -1);
+    int identity_map(hipStream_t s);   // sc_map_ of a full build (leaf i: i), built when something reads it
     static int multi_materialize(Volume* const* v, int G, const Exec& ex, int* failed);
     static int multi_apron(Volume* const* v, int G, int chan, float boundval, const Exec& ex, int* failed);
     static int multi_render(Volume* const* v, int G, const int* shading, const int* chan, const int* buf, const Exec& ex,
@@ -252,6 +254,14 @@ private:
     hipEvent_t bounds_ev_ = nullptr;
     hipEvent_t small_ev_ = nullptr;   // InsertPointsSubcell's early readback of its small words
     int resolve_bounds();
+    // Facts of a full build, valid while full_gen_ equals topo_gen_: every
+    // leaf is in use and linked (so slot and subcell block of leaf i are i),
+    // and, when full_box_, the box of the leaves.
+    unsigned full_gen_ = ~0u;
+    bool full_box_ = false;
+    float full_min_[3] = {0, 0, 0}, full_max_[3] = {0, 0, 0};
+    bool all_leaves() const { return full_gen_ == topo_gen_ && !dev_stale_; }
+    void note_full_build(const float* mnmx, bool odd, float radius, const BitDomain& d0);
     float epsilon_ = 0.001f;
     int maxiter_ = 256;
 
@@ -288,6 +298,7 @@ private:
     DevBuf bkt_key_, bkt_slot_, bkt_cnt_, bkt_off_, sorted_;
     int sc_len_ = 0, num_sc_ = 0, sc_bricks_ = 0, sc_map_n_ = 0;
     bool last_insert_pull_ = false;
+    bool map_ready_ = false;       // sc_map_ holds the current insert's mapping (built on demand otherwise)
     bool entries_stale_ = false;   // pull insert done, subcell tables not built yet
     // InsertPointsSubcell_FP16: u16 entries (3 per entry) and the bounds they
     // are quantised against; valid until the next insert
