@@ -35,7 +35,7 @@ __device__ inline void k_neighbors_body(const NbrArgs& a, uint32_t bid, uint32_t
     int v = -1;
     if (a.bcnt) {
         if (b < a.n && d < a.spb) a.bcnt[u64(b) * u64(a.spb) + u64(d)] = 0;
-        if (g < 64) a.lenparts[g] = 0;
+        if (g < 96) a.lenparts[g] = 0;
         if (g == 0) *a.orphans = 0;
     }
     if (valid) {

@@ -355,7 +355,7 @@ struct BucketArgs {
     // would make (u64 counter); needs the neighbour masks and R <= spd
     const uint32_t* nmask;
     float radius;
-    u64* len;             // 64 partial counters, summed by launch_sum_parts_multi
+    u64* len;             // 64 partial counters, summed by launch_sum_parts_multi, then 64 u32 with the fullest subcells' points
     int rule;             // BIN_FLOAT or BIN_FP16
     BrickTab bt;          // leaf lookup (tab == nullptr: the walk)
 };
@@ -364,6 +364,7 @@ struct SumArgs {
     u64* out;
     const uint32_t* orphans;
     uint32_t* orphans_out;   // or null
+    uint32_t* fullest_out;   // points of the fullest subcell; or null
 };
 hipError_t launch_sum_parts_multi(const SumArgs* a, int G, Arena* ar, hipStream_t s);
 hipError_t launch_bucket_points_multi(const BucketArgs* a, int G, Arena* ar, hipStream_t s);
@@ -416,6 +417,11 @@ struct BucketGatherArgs {
     int accumulate;
     void* faces;          // optional (scatter kernel): the six 8x8 boundary faces of each brick, channel type
     int levelset;         // 1: GatherLevelSet (nearest-entry kernel)
+    // scatter gathers: the bricks left to the dense kernel (count, workgroups
+    // done, leaf indices; the first two zero between launches)
+    uint32_t* heavy;
+    uint32_t fullest;     // no subcell holds more points than this
+    uint32_t dense_cell;  // bricks with more candidates a cell than this are dense
 };
 hipError_t launch_bucket_gather_multi(const BucketGatherArgs* a, int G, Arena* ar, hipStream_t s);
 
@@ -454,7 +460,8 @@ struct NbrArgs {
     long long* base;      // optional: atlas offset of each neighbour's brick (d = 13: own), -1 if none
     BrickTab bt;          // leaf lookup (tab == nullptr: the walks)
     // optional (an insert follows): the brick's spb bucket counters, the 64
-    // partial entry counts and the orphan count, set to zero
+    // partial entry counts with the 64 words behind them and the orphan count,
+    // set to zero
     uint32_t* bcnt;
     int spb;
     u64* lenparts;

@@ -141,7 +141,7 @@ Volume::~Volume() {
         for (int l = 0; l < MAXLEV; l++) pool_[g][l].dev.release();
     for (auto& c : chan_) c.data.release();
     for (auto& r : rbuf_) r.data.release();
-    DevBuf* bufs[] = {&amap_, &nbr_, &nmask_, &nbase_, &faces_, &lenparts_, &pts_owned_, &clr_owned_, &sc_cnt_, &sc_off_, &sc_pos_, &sc_nid_, &sc_map_, &sc_pnt_, &sc_use_,
+    DevBuf* bufs[] = {&amap_, &nbr_, &nmask_, &nbase_, &faces_, &heavy_, &lenparts_, &pts_owned_, &clr_owned_, &sc_cnt_, &sc_off_, &sc_pos_, &sc_nid_, &sc_map_, &sc_pnt_, &sc_use_,
                       &bkt_key_, &bkt_slot_, &bkt_cnt_, &bkt_off_, &sorted_, &sc_flags_, &small_, &masks_, &bitmaps_, &ranks_, &scan_tmp_, &flags_, &slot_scan_, &tf_dev,
                       &incr_marker_, &sc_pnt16_, &view_dev_, &view_scene_, &kb_keys_, &kb_keysB_, &kb_cnt_, &kb_off_,
                       &kb_tmp_, &kb_hist_, &kb_flags_, &kb_pos_, &kb_list_, &btab_, &bbox_part_};
@@ -852,7 +852,7 @@ unsigned long long Volume::device_bytes() const {
         for (int l = 0; l < MAXLEV; l++) b += pool_[g][l].dev.bytes;
     for (const auto& c : chan_) b += c.data.bytes;
     for (const auto& r : rbuf_) b += r.data.bytes;
-    const DevBuf* bufs[] = {&amap_, &nbr_, &nmask_, &nbase_, &faces_, &lenparts_, &pts_owned_, &sc_cnt_, &sc_off_, &sc_pos_, &sc_nid_, &sc_map_, &sc_pnt_,
+    const DevBuf* bufs[] = {&amap_, &nbr_, &nmask_, &nbase_, &faces_, &heavy_, &lenparts_, &pts_owned_, &sc_cnt_, &sc_off_, &sc_pos_, &sc_nid_, &sc_map_, &sc_pnt_,
                             &sc_use_, &bkt_key_, &bkt_slot_, &bkt_cnt_, &bkt_off_, &sorted_, &sc_flags_, &small_,
                             &masks_, &bitmaps_, &ranks_, &scan_tmp_, &flags_, &slot_scan_, &tf_dev,
                       &incr_marker_, &sc_pnt16_, &view_dev_, &view_scene_, &kb_keys_, &kb_keysB_, &kb_cnt_, &kb_off_,

@@ -64,7 +64,7 @@ struct SharedStream {
 static const int SMALL_WORDS = 64;
 // small per-grid result words (device dsmall / pinned hsmall, SMALL_WORDS each)
 enum { SM_BBOX = 0, SM_LINKED = 8, SM_TOTAL = 9, SM_ORPHANS = 10, SM_BUCKETS = 11, SM_LEN = 12, SM_COUNTS = 16, SM_BOUNDS = 40,
-       SM_UNFLAGGED = 48 };
+       SM_UNFLAGGED = 48, SM_FULLEST = 49 };
 struct Graph;
 struct Exec {
     hipStream_t s;
@@ -278,6 +278,7 @@ private:
     // The scatter gather's copy of each brick's boundary faces, current while
     // nothing else has written the atlas (atlas_epoch_ counts atlas writes).
     DevBuf faces_;
+    DevBuf heavy_;      // bricks the scatter gather leaves to the dense one (BucketGatherArgs::heavy)
     unsigned atlas_epoch_ = 0, faces_epoch_ = ~0u, faces_topo_ = ~0u;
     int faces_chan_ = -1;
     unsigned nbr_gen_ = ~0u;
@@ -307,6 +308,8 @@ private:
     float q_min_[3] = {0, 0, 0}, q_range_[3] = {0, 0, 0};
     int bkt_scs_ = 0, bkt_R_ = 0;
     float bkt_radius_ = 0.f;
+    int bkt_n_ = 0;                // points of the insert
+    uint32_t bkt_fullest_ = ~0u;   // points of the fullest subcell (~0: not known)
     unsigned bkt_gen_ = ~0u;       // topology generation of the current buckets
 
     // topology scratch
