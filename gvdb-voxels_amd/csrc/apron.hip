@@ -133,12 +133,9 @@ static float apron_bound_u8x4(float b) {
 
 // Apron voxel a of a padded brick of side br = w + 2: the two z faces
 // (br^2 each), then per interior z layer its ring (br^2 - w^2: the y = 0 and
-// y = br - 1 rows, then x = 0 / x = br - 1 of each row between).  W > 0: the
-// brick width known when compiled (its divisions become multiplies).
-template <int W>
-__device__ inline void apron_decode(int a, int w_rt, int& x, int& y, int& z) {
-    const unsigned w = W > 0 ? unsigned(W) : unsigned(w_rt);
-    const unsigned br = w + 2, face = br * br, ring = br * br - w * w, u = unsigned(a);
+// y = br - 1 rows, then x = 0 / x = br - 1 of each row between).
+__host__ __device__ constexpr void apron_decode(int a, int w_, int& x, int& y, int& z) {
+    const unsigned w = unsigned(w_), br = w + 2, face = br * br, ring = br * br - w * w, u = unsigned(a);
     if (u < 2 * face) {
         z = u < face ? 0 : int(br) - 1;
         const unsigned r = u < face ? u : u - face;
@@ -154,75 +151,97 @@ __device__ inline void apron_decode(int a, int w_rt, int& x, int& y, int& z) {
     }
 }
 
-// Apron voxel `a` (0..487) of brick b, given the atlas offsets of the brick
-// and its 26 neighbours (-1: none).  Enumeration: the z = 0 and z = 9 faces
-// (100 each), then the 36-voxel rings of z = 1..8.
-template <typename AT>
-__device__ inline void apron_voxel(const ApronArgs& ap, int b, int a, const long long* base) {
-    const Tree& t = ap.t;
-    AT* atlas = reinterpret_cast<AT*>(ap.atlas);
-    const int br = t.brick_res;        // 10
-    const int w = t.brickwid;          // 8
-    int x, y, z;
-    if (w == 8) apron_decode<8>(a, w, x, y, z);   // uniform: the usual 8^3 bricks
-    else apron_decode<0>(a, w, x, y, z);
-    int dx = x == 0 ? -1 : (x == br - 1 ? 1 : 0);
-    int dy = y == 0 ? -1 : (y == br - 1 ? 1 : 0);
-    int dz = z == 0 ? -1 : (z == br - 1 ? 1 : 0);
-    const int d = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1);
-    const long long nbase = base[d];
-    const u64 own = u64(base[13]) + u64((z * br + y) * br + x);
-    float v = ap.boundval;
-    if (nbase >= 0) {
-        // interior coordinate inside the neighbour
-        const int sx = (x - 1) - dx * w, sy = (y - 1) - dy * w, sz = (z - 1) - dz * w;
-        if (ap.faces) {
-            // it lies on the neighbour's face towards this brick (x face first)
-            const int f = dx ? (dx < 0 ? 1 : 0) : (dy ? (dy < 0 ? 3 : 2) : (dz < 0 ? 5 : 4));
-            const int i = dx ? sz * 8 + sy : (dy ? sz * 8 + sx : sy * 8 + sx);
-            const int nb = ap.nbr[u64(b) * 27 + d];
-            v = ld<AT>(reinterpret_cast<const AT*>(ap.faces), u64(nb) * FACE_VALS + u64(f * 64 + i));
-        } else {
-            v = ld<AT>(atlas, u64(nbase) + u64(((sz + 1) * br + sy + 1) * br + sx + 1));
+// Where apron voxel a of a brick w wide lies (own: its index in the padded
+// brick) and where its value is: direction d of the neighbour, and the index
+// in that neighbour's padded brick (faces = false) or among its six face
+// layers (true: the face towards this brick, x faces first).
+__host__ __device__ constexpr void apron_source(int a, int w, bool faces, int& own, int& d, int& src) {
+    int x = 0, y = 0, z = 0;
+    apron_decode(a, w, x, y, z);
+    const int br = w + 2;
+    const int dx = x == 0 ? -1 : (x == br - 1 ? 1 : 0), dy = y == 0 ? -1 : (y == br - 1 ? 1 : 0),
+              dz = z == 0 ? -1 : (z == br - 1 ? 1 : 0);
+    own = (z * br + y) * br + x;
+    d = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1);
+    const int sx = (x - 1) - dx * w, sy = (y - 1) - dy * w, sz = (z - 1) - dz * w;   // interior voxel of the neighbour
+    if (faces)
+        src = dx ? (dx < 0 ? 1 : 0) * 64 + sz * 8 + sy
+                 : (dy ? (dy < 0 ? 3 : 2) * 64 + sz * 8 + sx : (dz < 0 ? 5 : 4) * 64 + sy * 8 + sx);
+    else
+        src = ((sz + 1) * br + sy + 1) * br + sx + 1;
+}
+
+// The same for 8^3 bricks as a table: own | d << 10 | src << 15.
+static const int APRON8 = 488;
+struct ApronTable {
+    uint32_t e[2][APRON8];
+};
+static constexpr ApronTable make_apron_table() {
+    ApronTable t{};
+    for (int f = 0; f < 2; f++)
+        for (int a = 0; a < APRON8; a++) {
+            int own = 0, d = 0, src = 0;
+            apron_source(a, 8, f != 0, own, d, src);
+            t.e[f][a] = uint32_t(own) | uint32_t(d) << 10 | uint32_t(src) << 15;
         }
-    }
-    st<AT>(atlas, own, v);
+    return t;
 }
+static __constant__ ApronTable apron_table = make_apron_table();
 
-// One 512-thread workgroup per brick; threads 0..487 each own one apron voxel
-// of the padded 10^3 brick (apron 1, 8^3 interior).
-template <typename AT>
-__device__ inline void k_apron_body(const ApronArgs& ap, uint32_t bid, uint32_t) {
-    __shared__ long long base[27];
-    const Tree& t = ap.t;
-    const int b = int(bid);
-    const int a = threadIdx.x;
-    const int br = t.brick_res, w = t.brickwid;
-    // atlas offsets of the brick and its 26 neighbours (-1: none), one load
-    if (a < 27) base[a] = ap.base[u64(b) * 27 + a];
-    __syncthreads();
-    if (a >= 2 * br * br + w * (br * br - w * w) || base[13] < 0) return;
-    apron_voxel<AT>(ap, b, a, base);
-}
-
-GVDB_MULTI_T(k_apron, typename AT, AT, ApronArgs, 512)
-
-// A run of up to RUN consecutive bricks b0.. of one grid, its voxels spread
-// over all 512 threads: the atlas offsets of the run's bricks in one load and
-// one barrier, then RUN * 488 voxels in turn (a workgroup per brick launched
-// eight waves for 488 one-voxel threads).  Ends with a barrier, so the next
-// run may reuse the offsets' LDS.
+// A run of up to RUN consecutive bricks b0.. of one grid.  The sources of the
+// run's 26 directions a brick (offset of the neighbour's faces or padded
+// brick, -1: none; 13: the brick's own offset) come in one load and one
+// barrier.  8^3 bricks: thread a owns apron voxel a of every brick of the run,
+// its place and its source looked up once, so a voxel costs an LDS read, a
+// load and a store, and the loads of eight bricks are in flight together
+// (decoding every voxel, and for faces a second lookup behind it, took most of
+// the time: 73 k bricks, FP32, 0.156 -> 0.126 ms).  What is left is the writes:
+// every row of a brick has apron voxels at both ends, so all of its cache
+// lines are written for half of their bytes.  Ends with a barrier, so the next
+// run may reuse the LDS.
 template <typename AT, int RUN>
-__device__ inline void apron_run(const ApronArgs& a0, uint32_t b0, long long* base) {
-    const int nb = min(RUN, int(uint32_t(a0.n) - b0));
-    for (int i = threadIdx.x; i < nb * 27; i += 512) base[i] = a0.base[u64(b0) * 27 + u64(i)];
+__device__ inline void apron_run(const ApronArgs& ap, uint32_t b0, long long* base) {
+    const int nb = min(RUN, int(uint32_t(ap.n) - b0));
+    AT* atlas = reinterpret_cast<AT*>(ap.atlas);
+    const AT* from = ap.faces ? reinterpret_cast<const AT*>(ap.faces) : atlas;
+    for (int i = threadIdx.x; i < nb * 27; i += 512) {
+        const u64 e = u64(b0) * 27 + u64(i);
+        long long o = ap.base[e];
+        if (ap.faces && o >= 0 && i % 27 != 13) o = (long long)ap.nbr[e] * FACE_VALS;
+        base[i] = o;
+    }
     __syncthreads();
-    const int br = a0.t.brick_res, w = a0.t.brickwid;
-    const int per = 2 * br * br + w * (br * br - w * w);
-    for (int v = threadIdx.x; v < nb * per; v += 512) {
-        const int k = w == 8 ? int(unsigned(v) / 488u) : v / per, a = v - k * per;   // 488 = per for 8^3 bricks
-        if (base[k * 27 + 13] < 0) continue;
-        apron_voxel<AT>(a0, int(b0) + k, a, base + k * 27);
+    const int w = ap.t.brickwid;
+    if (w == 8) {
+        if (threadIdx.x < APRON8) {
+            const uint32_t t = apron_table.e[ap.faces ? 1 : 0][threadIdx.x];
+            const int own = int(t & 1023u), d = int((t >> 10) & 31u), src = int(t >> 15);
+            for (int k0 = 0; k0 < nb; k0 += 8) {
+                float v[8];
+                long long at[8];
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    at[k] = k0 + k < nb ? base[(k0 + k) * 27 + 13] : -1ll;
+                    const long long o = at[k] >= 0 ? base[(k0 + k) * 27 + d] : -1ll;
+                    v[k] = ap.boundval;
+                    if (o >= 0) v[k] = ld<AT>(from, u64(o) + u64(src));
+                }
+#pragma unroll
+                for (int k = 0; k < 8; k++)
+                    if (at[k] >= 0) st<AT>(atlas, u64(at[k]) + u64(own), v[k]);
+            }
+        }
+    } else {
+        const int br = ap.t.brick_res;
+        const int per = 2 * br * br + w * (br * br - w * w);
+        for (int v = threadIdx.x; v < nb * per; v += 512) {
+            const int k = v / per;
+            if (base[k * 27 + 13] < 0) continue;
+            int own = 0, d = 0, src = 0;
+            apron_source(v - k * per, w, ap.faces != nullptr, own, d, src);
+            const long long o = base[k * 27 + d];
+            st<AT>(atlas, u64(base[k * 27 + 13]) + u64(own), o >= 0 ? ld<AT>(from, u64(o) + u64(src)) : ap.boundval);
+        }
     }
     __syncthreads();
 }
@@ -300,7 +319,7 @@ static void launch_apron_seq(int run, dim3 grid, hipStream_t s, const ApronArgs&
     case 8: hipLaunchKernelGGL((k_apron_flat<AT, 8>), grid, dim3(512), 0, s, a0, m); break;
     case 16: hipLaunchKernelGGL((k_apron_flat<AT, 16>), grid, dim3(512), 0, s, a0, m); break;
     case 32: hipLaunchKernelGGL((k_apron_flat<AT, 32>), grid, dim3(512), 0, s, a0, m); break;
-    default: hipLaunchKernelGGL(k_apron<AT>, grid, dim3(512), 0, s, a0, m); break;
+    default: hipLaunchKernelGGL((k_apron_flat<AT, 1>), grid, dim3(512), 0, s, a0, m); break;
     }
 }
 
@@ -340,7 +359,12 @@ hipError_t launch_apron_multi(const ApronArgs* a, int G, Arena* ar, hipStream_t 
         hipError_t e = multi_setup(ar, sel.data(), nb.data(), int(sel.size()), s, L);
         if (e != hipSuccess) return e;
         if (L.blocks == 0) continue;
-        L.map.xcd = knob(KNOB_XCD_ORDER);
+        // without the compact layers a brick reads rows of its neighbours' lines:
+        // each XCD takes a contiguous part, so those stay in its L2 (17 k bricks
+        // 0.0365 -> 0.0273 ms; with them the order does not matter)
+        bool rows = true;
+        for (const ApronArgs& x : sel) rows = rows && !x.faces;
+        L.map.xcd = rows ? 1 : knob(KNOB_XCD_ORDER);
         uint32_t* ctr = nullptr;
         const uint32_t nwg = std::min<uint32_t>(L.blocks, APRON_QUEUE_WORKGROUPS);
         if (queue) {
@@ -405,14 +429,17 @@ hipError_t launch_apron_noalloc(const Tree& t, void* sp, const void* faces, void
     hipLaunchKernelGGL(k_neighbors, dim3(uint32_t((u64(bricks) * 32 + 255) / 256)), dim3(256), 0, s, na, one);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
+    const dim3 grid(uint32_t((bricks + 7) / 8));
+    MultiMap order = one;   // as launch_apron_multi orders the workgroups
+    if (!faces || atlas_type == T_UCHAR4) order.xcd = 1;
     if (atlas_type == T_UCHAR4) {
         const ApronArgs aa{t, base, nbr, nullptr, atlas, atlas_type, apron_bound_u8x4(boundval), bricks};
-        hipLaunchKernelGGL(k_apron<uint32_t>, dim3(uint32_t(bricks)), dim3(512), 0, s, aa, one);
+        hipLaunchKernelGGL((k_apron_flat<uint32_t, 8>), grid, dim3(512), 0, s, aa, order);
         return hipGetLastError();
     }
     const ApronArgs aa{t, base, nbr, faces, atlas, atlas_type, boundval, bricks};
-    if (atlas_type == T_HALF) hipLaunchKernelGGL(k_apron<__half>, dim3(uint32_t(bricks)), dim3(512), 0, s, aa, one);
-    else hipLaunchKernelGGL(k_apron<float>, dim3(uint32_t(bricks)), dim3(512), 0, s, aa, one);
+    if (atlas_type == T_HALF) hipLaunchKernelGGL((k_apron_flat<__half, 8>), grid, dim3(512), 0, s, aa, order);
+    else hipLaunchKernelGGL((k_apron_flat<float, 8>), grid, dim3(512), 0, s, aa, order);
     return hipGetLastError();
 }
 
