@@ -207,7 +207,8 @@ __device__ inline void apron_run(const ApronArgs& ap, uint32_t b0, long long* ba
     for (int i = threadIdx.x; i < nb * 27; i += 512) {
         const u64 e = u64(b0) * 27 + u64(i);
         long long o = ap.base[e];
-        if (ap.faces && o >= 0 && i % 27 != 13) o = (long long)ap.nbr[e] * FACE_VALS;
+        if (ap.faces && o >= 0 && i % 27 != 13)
+            o = (ap.by_slot ? (long long)(u64(o) / u64(ap.t.brick_vox)) : (long long)ap.nbr[e]) * FACE_VALS;
         base[i] = o;
     }
     __syncthreads();

@@ -251,6 +251,16 @@ struct ComputeArgs {
     int op;
     float p1, p2, p3;
     int slots;            // smooth/noise/grow: atlas slots 0 .. slots-1
+    double inv;           // smooth: 1 / (p1 + 6) where that is a power of two, else 0
+    // an iteration of a smoothing with the apron refreshed in between:
+    int from_cells, to_cells;   // the interior voxels come from / go to `cells` (512 a slot), else the atlas
+    void* cells;
+    const void* faces_in;       // the slots' boundary layers (FACE_VALS a slot) before and after
+    void* faces_out;            // (optional)
+    int* links;                 // 8 a slot: where the voxels beyond each layer come from
+    const long long* base;      // the neighbour pass's brick offsets, `leaves` rows
+    int leaves;
+    float boundval;
     int lo[3], hi[3];     // fill: inclusive atlas-voxel range
 };
 hipError_t launch_compute(const ComputeArgs& a, hipStream_t s);
@@ -478,6 +488,7 @@ struct ApronArgs {
     int atlas_type;
     float boundval;
     int n;
+    int by_slot;             // `faces` is indexed by atlas slot, not by leaf
 };
 hipError_t launch_apron_multi(const ApronArgs* a, int G, Arena* ar, hipStream_t s);
 

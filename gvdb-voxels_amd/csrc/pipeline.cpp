@@ -1262,7 +1262,8 @@ int Volume::multi_gather(Volume* const* vs, int G, int scs, const int* len, cons
 }
 
 // ----------------------------------------------------------- UpdateApron ----
-int Volume::multi_apron(Volume* const* vs, int G, int c, float boundval, const Exec& ex, int* failed) {
+int Volume::multi_apron(Volume* const* vs, int G, int c, float boundval, const Exec& ex, int* failed,
+                        const void* slot_faces) {
     // UpdateApron (gvdb_volume_gvdb.cpp:4418-4457)
     std::vector<NbrArgs> na;
     std::vector<FillArgs> nf;
@@ -1289,8 +1290,9 @@ int Volume::multi_apron(Volume* const* vs, int G, int c, float boundval, const E
             v->nbr_gen_ = v->topo_gen_;
         }
         const bool faces = v->faces_chan_ == c && v->faces_epoch_ == v->atlas_epoch_ && v->faces_topo_ == v->topo_gen_;
-        aa.push_back(ApronArgs{t, v->nbase_.as<long long>(), v->nbr_.as<int>(), faces ? v->faces_.p : nullptr,
-                               v->chan_[c].data.p, v->chan_[c].type, boundval, bricks});
+        aa.push_back(ApronArgs{t, v->nbase_.as<long long>(), v->nbr_.as<int>(),
+                               slot_faces ? slot_faces : (faces ? v->faces_.p : nullptr), v->chan_[c].data.p,
+                               v->chan_[c].type, boundval, bricks, slot_faces ? 1 : 0});
     }
     if (aa.empty()) return GVDB_OK;
     Volume* v0 = vs[0];

@@ -141,7 +141,7 @@ Volume::~Volume() {
         for (int l = 0; l < MAXLEV; l++) pool_[g][l].dev.release();
     for (auto& c : chan_) c.data.release();
     for (auto& r : rbuf_) r.data.release();
-    DevBuf* bufs[] = {&amap_, &nbr_, &nmask_, &nbase_, &faces_, &heavy_, &lenparts_, &pts_owned_, &clr_owned_, &sc_cnt_, &sc_off_, &sc_pos_, &sc_nid_, &sc_map_, &sc_pnt_, &sc_use_,
+    DevBuf* bufs[] = {&amap_, &nbr_, &nmask_, &nbase_, &faces_, &layers_, &heavy_, &lenparts_, &pts_owned_, &clr_owned_, &sc_cnt_, &sc_off_, &sc_pos_, &sc_nid_, &sc_map_, &sc_pnt_, &sc_use_,
                       &bkt_key_, &bkt_slot_, &bkt_cnt_, &bkt_off_, &sorted_, &sc_flags_, &small_, &masks_, &bitmaps_, &ranks_, &scan_tmp_, &flags_, &slot_scan_, &tf_dev,
                       &incr_marker_, &sc_pnt16_, &view_dev_, &view_scene_, &kb_keys_, &kb_keysB_, &kb_cnt_, &kb_off_,
                       &kb_tmp_, &kb_hist_, &kb_flags_, &kb_pos_, &kb_list_, &btab_, &bbox_part_};
@@ -776,15 +776,62 @@ int Volume::compute(int effect, int c, int iterations, const float p[3], bool up
         a.lo[k] = 1;
         a.hi[k] = std::min(8 * blocks, res - 1);
     }
+    if (effect == OP_SMOOTH) {
+        int e = 0;
+        const double d = double(a.p1) + 6.0;
+        a.inv = std::fabs(std::frexp(d, &e)) == 0.5 && e > -1000 && e < 1000 ? 1.0 / d : 0.0;
+    }
+    // noise and grow read no neighbour: only the last apron is seen
+    const bool pointwise = effect == OP_NOISE || effect == OP_GROW;
     for (int it = 0; it < iterations; it++) {
+        if (update_apron_each && effect == OP_SMOOTH && iterations - it >= 2 && smooth_layers(a, c, iterations - it, boundval, rc))
+            return rc;
         HIPCHK(launch_compute(a, stream));
         atlas_epoch_++;
-        if (update_apron_each) {
+        if (update_apron_each && !(pointwise && it + 1 < iterations)) {
             rc = update_apron(c, boundval);
             if (rc) return rc;
         }
     }
     return GVDB_OK;
+}
+
+// The smoothing's remaining `n` iterations with one apron at the end
+// (compute.hip); false where the neighbour table is not current (the first
+// iteration's apron builds it) or there is no room for the workspace, at most
+// LAYERS_MAX bytes, 840 k bricks in FP32 (then each iteration writes its apron).
+bool Volume::smooth_layers(ComputeArgs a, int c, int n, float boundval, int& rc) {
+    static const size_t LAYERS_MAX = size_t(4) << 30;
+    if (brickwid_ != 8 || a.slots <= 0 || atlas_gen_ != topo_gen_ || nbr_gen_ != topo_gen_) return false;
+    const size_t e = chan_[c].elem(), slots = size_t(a.slots);
+    const size_t cells = slots * 512 * e, layer = slots * FACE_VALS * e, need = cells + 2 * layer + slots * 8 * sizeof(int);
+    if (need > LAYERS_MAX) return false;
+    if (layers_.ensure(need) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    char* p = layers_.as<char>();
+    char* face[2] = {p + cells, p + cells + layer};
+    a.cells = p;
+    a.links = reinterpret_cast<int*>(p + cells + 2 * layer);
+    a.base = nbase_.as<long long>();
+    a.leaves = int(pool_[0][0].lastEle);
+    a.boundval = boundval;
+    for (int it = 0; it < n; it++) {
+        a.from_cells = it > 0;
+        a.to_cells = it + 1 < n;
+        a.faces_in = face[(it + 1) & 1];
+        a.faces_out = face[it & 1];
+        const hipError_t err = launch_compute(a, stream);
+        if (err != hipSuccess) {
+            rc = hip_fail(err, "Compute");
+            return true;
+        }
+    }
+    atlas_epoch_++;
+    Volume* v = this;
+    rc = multi_apron(&v, 1, c, boundval, self_exec(), nullptr, a.faces_out);
+    return true;
 }
 
 int Volume::update_apron(int c, float boundval) {
@@ -852,7 +899,7 @@ unsigned long long Volume::device_bytes() const {
         for (int l = 0; l < MAXLEV; l++) b += pool_[g][l].dev.bytes;
     for (const auto& c : chan_) b += c.data.bytes;
     for (const auto& r : rbuf_) b += r.data.bytes;
-    const DevBuf* bufs[] = {&amap_, &nbr_, &nmask_, &nbase_, &faces_, &heavy_, &lenparts_, &pts_owned_, &sc_cnt_, &sc_off_, &sc_pos_, &sc_nid_, &sc_map_, &sc_pnt_,
+    const DevBuf* bufs[] = {&amap_, &nbr_, &nmask_, &nbase_, &faces_, &layers_, &heavy_, &lenparts_, &pts_owned_, &sc_cnt_, &sc_off_, &sc_pos_, &sc_nid_, &sc_map_, &sc_pnt_,
                             &sc_use_, &bkt_key_, &bkt_slot_, &bkt_cnt_, &bkt_off_, &sorted_, &sc_flags_, &small_,
                             &masks_, &bitmaps_, &ranks_, &scan_tmp_, &flags_, &slot_scan_, &tf_dev,
                       &incr_marker_, &sc_pnt16_, &view_dev_, &view_scene_, &kb_keys_, &kb_keysB_, &kb_cnt_, &kb_off_,

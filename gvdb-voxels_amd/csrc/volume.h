@@ -105,6 +105,7 @@ public:
     int accumulate_topology(int n, float radius, const float orig[3], int min_depth);
     int compute(int effect, int chan, int iterations, const float params[3], bool update_apron, bool skip_aprons,
                 float boundval);
+    bool smooth_layers(ComputeArgs a, int chan, int n, float boundval, int& rc);
     // VBX files (vbx.cpp)
     int save_vbx(const char* path);
     int load_vbx(const char* path, int force_major, int force_minor);
@@ -219,7 +220,8 @@ public:
                             bool levelset, const Exec& ex, int* failed, bool fp16 = false, int chanC = -1);
     int identity_map(hipStream_t s);   // sc_map_ of a full build (leaf i: i), built when something reads it
     static int multi_materialize(Volume* const* v, int G, const Exec& ex, int* failed);
-    static int multi_apron(Volume* const* v, int G, int chan, float boundval, const Exec& ex, int* failed);
+    static int multi_apron(Volume* const* v, int G, int chan, float boundval, const Exec& ex, int* failed,
+                           const void* slot_faces = nullptr);
     static int multi_render(Volume* const* v, int G, const int* shading, const int* chan, const int* buf, const Exec& ex,
                             int* failed);
     int hip_fail(hipError_t e, const char* what);
@@ -278,6 +280,7 @@ private:
     // The scatter gather's copy of each brick's boundary faces, current while
     // nothing else has written the atlas (atlas_epoch_ counts atlas writes).
     DevBuf faces_;
+    DevBuf layers_;     // smoothing: interior voxels, two sets of boundary layers and their links, by slot
     DevBuf heavy_;      // bricks the scatter gather leaves to the dense one (BucketGatherArgs::heavy)
     unsigned atlas_epoch_ = 0, faces_epoch_ = ~0u, faces_topo_ = ~0u;
     int faces_chan_ = -1;

@@ -1,0 +1,37 @@
+"""Smoothing of several iterations with the apron refreshed in between
+(Compute, src/gvdb_volume_gvdb.cpp:4527-4552 of the reference) keeps the
+bricks' boundary layers and writes one apron at the end; the result has to be
+that of single iterations, bit by bit: atlases of a few bricks, of an odd number
+of bricks, float and half, a boundary value, and a divisor that is no power of
+two.  Noise and grow, which read no neighbour, likewise write only the last
+apron."""
+import numpy as np
+import pytest
+
+import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("effect,params", [(113, (2.0, 0.0, 0.0)), (113, (0.3, 0.05, 0.0)), (114, (0.3, 0.0, 0.0)),
+                                           (115, (0.05, 0.0, 0.0))])
+@pytest.mark.parametrize("half,boundval,n,iters", [(False, 0.0, 3000, 2), (False, 0.75, 3000, 3), (True, 0.3, 3000, 4),
+                                                   (False, 0.5, 2, 2), (True, 0.0, 60000, 5)])
+def test_iterations_in_one_call_equal_single_calls(gpu, effect, params, half, boundval, n, iters):
+    from gvdb_amd import workloads as W
+    import gvdb_amd as G
+    pts = W.sphere_shell(n, seed=17) if n > 2 else np.array([[60.5, 60.5, 60.5], [70.5, 73.5, 60.5]], np.float32)
+    out = []
+    for once in (True, False):
+        v, _ = H.gpu_volume(gpu, pts, 2.0, atlas_type=G.T_HALF if half else None, boundval=boundval)
+        if once:
+            v.Compute(effect, 0, iters, params, True, True, boundval)
+        else:
+            for _ in range(iters):
+                v.Compute(effect, 0, 1, params, True, True, boundval)
+        v.synchronize()
+        a = v.atlas(0, np.float16 if half else np.float32)
+        out.append(a[H.used_brick_mask(a.shape, v.atlas_map(), v.atlas_info()["cnt"])].copy())
+        v.close()
+    a, b = (x.view(np.uint16 if half else np.uint32) for x in out)
+    assert np.array_equal(a, b), "%d voxels differ" % int((a != b).sum())
