@@ -365,16 +365,17 @@ struct BucketArgs {
     // would make (u64 counter); needs the neighbour masks and R <= spd
     const uint32_t* nmask;
     float radius;
-    u64* len;             // 64 partial counters, summed by launch_sum_parts_multi, then 64 u32 with the fullest subcells' points
+    u64* len;             // 64 partial counters, summed by launch_sum_parts_multi, then 64 u32, one set where a subcell holds more than dense_cell points
     int rule;             // BIN_FLOAT or BIN_FP16
     BrickTab bt;          // leaf lookup (tab == nullptr: the walk)
+    uint32_t dense_cell;  // the gather's line (BucketGatherArgs)
 };
 struct SumArgs {
     const u64* parts;
     u64* out;
     const uint32_t* orphans;
     uint32_t* orphans_out;   // or null
-    uint32_t* fullest_out;   // points of the fullest subcell; or null
+    uint32_t* dense_out;     // whether a subcell holds more than dense_cell points; or null
 };
 hipError_t launch_sum_parts_multi(const SumArgs* a, int G, Arena* ar, hipStream_t s);
 hipError_t launch_bucket_points_multi(const BucketArgs* a, int G, Arena* ar, hipStream_t s);
@@ -430,7 +431,7 @@ struct BucketGatherArgs {
     // scatter gathers: the bricks left to the dense kernel (count, workgroups
     // done, leaf indices; the first two zero between launches)
     uint32_t* heavy;
-    uint32_t fullest;     // no subcell holds more points than this
+    uint32_t fullest;     // no subcell holds more points than this (~0: not known)
     uint32_t dense_cell;  // bricks with more candidates a cell than this are dense
 };
 hipError_t launch_bucket_gather_multi(const BucketGatherArgs* a, int G, Arena* ar, hipStream_t s);

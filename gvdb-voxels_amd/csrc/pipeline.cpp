@@ -803,6 +803,15 @@ int Volume::multi_clear_channel(Volume* const* vs, int G, int c, const Exec& ex,
 }
 
 // --------------------------------------------------- InsertPointsSubcell ----
+// The line above which a brick is the dense gather's, in points a cell of 64
+// voxels: 64, and twice the grid's own mean (the scatter kernel does as well
+// where all bricks are alike: 4 M points at one a voxel 0.305 ms there, 0.353
+// with a line at 64; 777 k clustered points take 0.238 ms with the line at 64,
+// 0.269 at 96, 0.215 at 32, where 1 M points at 0.7 a voxel go from 0.105 to 0.22)
+static uint32_t dense_cell(u64 points, u64 bricks) {
+    return std::max<uint32_t>(64u, uint32_t(points / (4 * std::max<u64>(bricks, 1))));
+}
+
 int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const float* radius, const float* trans3,
                          int* len, const Exec& ex, int* failed, int rule) {
     // InsertPointsSubcell (gvdb_volume_gvdb.cpp:4971-5092); with rule BIN_FP16
@@ -945,10 +954,11 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
             u64 nb = pl.numMap * u64(pl.spb);
             ba.push_back(BucketArgs{pl.t, pl.P, scs, pl.spb, {tr[0], tr[1], tr[2]}, v->bkt_key_.as<uint32_t>(),
                                     v->bkt_slot_.as<uint32_t>(), v->bkt_cnt_.as<uint32_t>(), small(g, SM_ORPHANS),
-                                    v->nmask_.as<uint32_t>(), radius[g], v->lenparts_.as<u64>(), rule, v->brick_tab()});
+                                    v->nmask_.as<uint32_t>(), radius[g], v->lenparts_.as<u64>(), rule, v->brick_tab(),
+                                    dense_cell(u64(n[g]), pl.numMap)});
             sums.push_back(SumArgs{v->lenparts_.as<u64>(), reinterpret_cast<u64*>(word(g, SM_LEN)),
                                    small(g, SM_ORPHANS), ex.cap ? nullptr : word(g, SM_ORPHANS),
-                                   ex.cap ? nullptr : word(g, SM_FULLEST)});
+                                   ex.cap ? nullptr : word(g, SM_DENSE)});
             sb.push_back(ScanArgs{v->bkt_cnt_.as<uint32_t>(), nullptr, 0, v->bkt_off_.as<uint32_t>(), nb, tmp2(g),
                                   small(g, SM_BUCKETS)});
             // SetPoints' colours travel with the bucketed points (fourth word)
@@ -1003,7 +1013,7 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
     for (int g = 0; g < G; g++) {
         Plan& pl = plan[g];
         pl.linked = pl.same ? uint32_t(pl.numMap) : ex.hsmall[g * SMALL_WORDS + SM_LINKED];
-        vs[g]->bkt_fullest_ = pl.pull ? ex.hsmall[g * SMALL_WORDS + SM_FULLEST] : ~0u;
+        vs[g]->bkt_fullest_ = pl.pull && !ex.hsmall[g * SMALL_WORDS + SM_DENSE] ? dense_cell(u64(n[g]), pl.numMap) : ~0u;
         pl.orphans = pl.pull ? ex.hsmall[g * SMALL_WORDS + SM_ORPHANS] : 0;
         {
             // the exact entry total in 64 bits (the u32 scan's wraps)
@@ -1198,13 +1208,7 @@ int Volume::multi_gather(Volume* const* vs, int G, int scs, const int* len, cons
                 }
                 bg.back().heavy = v->heavy_.as<uint32_t>();
                 bg.back().fullest = v->bkt_fullest_;
-                // dense: above 64 points a cell of 64 voxels, and twice the
-                // grid's own mean (the scatter kernel does as well where all
-                // bricks are alike: 4 M points at one a voxel 0.305 ms there,
-                // 0.353 with a line at 64; 777 k clustered points take 0.238 ms
-                // with the line at 64, 0.269 at 96, 0.215 at 32, where 1 M
-                // points at 0.7 a voxel go from 0.105 to 0.22)
-                bg.back().dense_cell = std::max<uint32_t>(64u, uint32_t(u64(v->bkt_n_) / (4 * v->pool_[0][0].lastEle)));
+                bg.back().dense_cell = dense_cell(u64(v->bkt_n_), v->pool_[0][0].lastEle);
             }
             continue;
         }

@@ -64,7 +64,7 @@ struct SharedStream {
 static const int SMALL_WORDS = 64;
 // small per-grid result words (device dsmall / pinned hsmall, SMALL_WORDS each)
 enum { SM_BBOX = 0, SM_LINKED = 8, SM_TOTAL = 9, SM_ORPHANS = 10, SM_BUCKETS = 11, SM_LEN = 12, SM_COUNTS = 16, SM_BOUNDS = 40,
-       SM_UNFLAGGED = 48, SM_FULLEST = 49 };
+       SM_UNFLAGGED = 48, SM_DENSE = 49 };
 struct Graph;
 struct Exec {
     hipStream_t s;
@@ -312,7 +312,7 @@ private:
     int bkt_scs_ = 0, bkt_R_ = 0;
     float bkt_radius_ = 0.f;
     int bkt_n_ = 0;                // points of the insert
-    uint32_t bkt_fullest_ = ~0u;   // points of the fullest subcell (~0: not known)
+    uint32_t bkt_fullest_ = ~0u;   // no subcell holds more points (~0: not known)
     unsigned bkt_gen_ = ~0u;       // topology generation of the current buckets
 
     // topology scratch
