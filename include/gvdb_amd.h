@@ -219,7 +219,7 @@ int gvdb_read_render_buf(gvdb_handle h, int buf, void* host_dst);
 #define GVDB_KNOB_RENDER_TILE_ISO 3
 #define GVDB_KNOB_GATHER_THREADS 4    /* threads per brick of the scatter gather, radius <= 3: 128, 256 */
 #define GVDB_KNOB_APRON_RUN 5         /* bricks per workgroup of the multi-grid apron: 1, 2, 4, 8 */
-#define GVDB_KNOB_XCD_ORDER 6         /* per-brick kernels: 0 launch order, 1 each XCD a contiguous range of bricks */
+#define GVDB_KNOB_XCD_ORDER 6         /* per-brick kernels: 0 launch order, 1 each XCD a contiguous range of bricks (always 1 for aprons that read whole bricks) */
 #define GVDB_KNOB_APRON_QUEUE 7       /* multi-grid apron: 0 static runs, 1 persistent workgroups over a brick queue */
 #define GVDB_KNOB_MARK_PATH 8         /* topology marks: 0 by domain size, 1 byte per brick, 2 direction masks, 3 bits,
                                          4 sorted brick keys (taken above 2^34 level-0 bricks) */
