@@ -1003,7 +1003,7 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
             v->bkt_radius_ = radius[g];
             v->bkt_n_ = n[g];
             v->bkt_gen_ = v->topo_gen_;
-            v->bkt_fullest_ = ~0u;   // every replay's points may differ
+            v->forget_fullest();
             ex.cap->inserts.push_back(Graph::Insert{v, ex.hsmall + size_t(g) * SMALL_WORDS});
         }
         return GVDB_OK;
@@ -1207,7 +1207,7 @@ int Volume::multi_gather(Volume* const* vs, int G, int scs, const int* len, cons
                     XCHK(v, launch_fill_u32(v->heavy_.as<uint32_t>(), 0u, 2, ex.s));
                 }
                 bg.back().heavy = v->heavy_.as<uint32_t>();
-                bg.back().fullest = v->bkt_fullest_;
+                bg.back().fullest = ex.cap ? ~0u : v->bkt_fullest_;   // a replay may follow any insert
                 bg.back().dense_cell = dense_cell(u64(v->bkt_n_), v->pool_[0][0].lastEle);
             }
             continue;

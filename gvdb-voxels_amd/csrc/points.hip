@@ -1270,7 +1270,8 @@ __device__ inline void k_push_gather_body(const BucketGatherArgs& a, uint32_t bi
     const float r = a.radius;
     const float r2cut = r * r * (1.0f + 0x1p-20f);
     const int span = 2 + 2 * a.R, ncell = span * span * span;
-    if (T > a.dense_cell * uint32_t(ncell)) {      // (uniform) k_dense_gather's
+    // (uniform) k_dense_gather's, by the record from which the host launches that one
+    if (a.fullest > a.dense_cell && T > u64(a.dense_cell) * unsigned(ncell)) {
         if (tid == 0) a.heavy[2 + atomicAdd(a.heavy, 1u)] = uint32_t(brick);
         return;
     }

@@ -67,6 +67,7 @@ int Volume::finish_recorded_insert(const uint32_t* slot) {
         return fail(GVDB_ERR_STATE, "graph replay: " + std::to_string(slot[SM_ORPHANS]) +
                                         " points fell outside the topology, which the recorded insert leaves out; "
                                         "rebuild the topology (or insert without the graph)");
+    forget_fullest();
     u64 total = 0;
     memcpy(&total, slot + SM_LEN, 8);
     if (total > 0x7FFFFFFFull) return fail(GVDB_ERR_RANGE, "graph replay: more than 2^31 subcell entries");

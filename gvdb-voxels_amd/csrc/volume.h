@@ -186,6 +186,8 @@ public:
     // after a replay: the recorded insert's readback (entry count, points
     // it could not place) into this grid's state
     int finish_recorded_insert(const uint32_t* slot);
+    // a recorded insert's points may differ at every replay
+    void forget_fullest() { bkt_fullest_ = ~0u; }
     // moves this grid's work to another stream (null: its own), ordered
     // after what is already queued, without waiting on the host
     int use_stream(const std::shared_ptr<SharedStream>& s);

@@ -113,3 +113,83 @@ def test_dense_bricks_half_batch_and_graph(gpu):
     gr.close()
     for x in vols + [v]:
         x.close()
+
+
+def _thin_and_dense(gpu):
+    """A grid over the union of two point sets of one size (one sparse, one
+    with dense bricks), its buffers grown by a chain of each, and what the
+    chain gives for each: (volume, {name: points}, {name: atlas}, {name: entries})."""
+    r = 2.0
+    dense = _points("full", 60000, 21)
+    g = np.random.default_rng(22)
+    thin = dense.copy()
+    thin[:60000] = (48.0 + 40.0 * g.random((60000, 3))).astype(np.float32)
+    sets = dict(thin=thin, dense=dense)
+    v = gpu.VolumeGVDB(0)
+    v.Configure(*H.TREE)
+    v.SetChannelDefault(16, 16, 1)
+    v.AddChannel(0, gpu.T_FLOAT, 1)
+    v.SetPoints(np.concatenate([thin, dense]))
+    v.RequestFullRebuild(True)
+    v.RebuildTopology(2 * len(thin), r, H.ZERO3)
+    v.FinishTopology(False, True)
+    v.UpdateAtlas()
+    atlas, entries = {}, {}
+    for k in ("dense", "thin"):
+        v.SetPoints(sets[k])
+        v.ClearChannel(0)
+        entries[k] = v.InsertPointsSubcell(4, len(thin), r, H.ZERO3)
+        v.GatherDensity(4, len(thin), r, H.ZERO3, entries[k], 0, 0, False)
+        v.UpdateApron(0, 0.0)
+        v.synchronize()
+        atlas[k] = v.atlas().view(np.uint32).copy()
+    assert not np.array_equal(atlas["thin"], atlas["dense"])
+    return v, sets, atlas, entries
+
+
+def test_recorded_gather_follows_later_inserts(gpu):
+    """GatherDensity and UpdateApron recorded alone, after an insert of sparse
+    points: every replay gathers what the last insert binned, dense bricks too."""
+    v, sets, atlas, entries = _thin_and_dense(gpu)
+    n = len(sets["thin"])
+    v.CaptureBegin()
+    v.GatherDensity(4, n, 2.0, H.ZERO3, entries["thin"], 0, 0, False)
+    v.UpdateApron(0, 0.0)
+    gr = v.CaptureEnd()
+    for k in ("dense", "thin", "dense", "dense"):
+        v.SetPoints(sets[k])
+        v.ClearChannel(0)
+        assert v.InsertPointsSubcell(4, n, 2.0, H.ZERO3) == entries[k]
+        gr.launch()
+        gr.synchronize()
+        assert np.array_equal(v.atlas().view(np.uint32), atlas[k]), k
+    gr.close()
+    v.close()
+
+
+@pytest.mark.parametrize("wait", [True, False])
+def test_eager_gather_after_a_replayed_insert(gpu, wait):
+    """The chain recorded; an eager insert of sparse points; a replay over
+    dense ones; then an eager gather (after the replay's wait or before it)."""
+    v, sets, atlas, entries = _thin_and_dense(gpu)
+    n = len(sets["thin"])
+    v.CaptureBegin()
+    v.InsertPointsSubcell(4, n, 2.0, H.ZERO3)
+    gr = v.CaptureEnd()
+    for _ in range(2):
+        v.SetPoints(sets["thin"])
+        ln = v.InsertPointsSubcell(4, n, 2.0, H.ZERO3)
+        assert ln == entries["thin"]
+        v.SetPoints(sets["dense"])
+        v.ClearChannel(0)
+        gr.launch()
+        if wait:
+            gr.synchronize()
+            ln = entries["dense"]
+        v.GatherDensity(4, n, 2.0, H.ZERO3, ln, 0, 0, False)
+        v.UpdateApron(0, 0.0)
+        v.synchronize()
+        gr.synchronize()
+        assert np.array_equal(v.atlas().view(np.uint32), atlas["dense"])
+    gr.close()
+    v.close()
