@@ -428,8 +428,8 @@ struct BucketGatherArgs {
     int accumulate;
     void* faces;          // optional (scatter kernel): the six 8x8 boundary faces of each brick, channel type
     int levelset;         // 1: GatherLevelSet (nearest-entry kernel)
-    // scatter gathers: the bricks left to the dense kernel (count, workgroups
-    // done, leaf indices; the first two zero between launches)
+    // scatter gathers: the bricks left to the dense kernel (count, then leaf
+    // indices), 1 + nleaves words; the launch empties it
     uint32_t* heavy;
     uint32_t fullest;     // no subcell holds more points than this (~0: not known)
     uint32_t dense_cell;  // bricks with more candidates a cell than this are dense

@@ -1200,12 +1200,7 @@ int Volume::multi_gather(Volume* const* vs, int G, int scs, const int* len, cons
                                           v->sorted_.as<float4>(), v->chan_[chanD].data.p, v->chan_[chanD].type,
                                           accum ? 1 : 0, faces, levelset ? 1 : 0, nullptr, ~0u, ~0u});
             if (!accum && !levelset) {
-                // (its two counters start at zero; the dense kernel clears them again)
-                const size_t words = size_t(v->pool_[0][0].lastEle) + 2;
-                if (v->heavy_.bytes < words * 4) {
-                    XCHK(v, v->heavy_.ensure(words * 4));
-                    XCHK(v, launch_fill_u32(v->heavy_.as<uint32_t>(), 0u, 2, ex.s));
-                }
+                XCHK(v, v->heavy_.ensure((size_t(v->pool_[0][0].lastEle) + 1) * 4));
                 bg.back().heavy = v->heavy_.as<uint32_t>();
                 bg.back().fullest = ex.cap ? ~0u : v->bkt_fullest_;   // a replay may follow any insert
                 bg.back().dense_cell = dense_cell(u64(v->bkt_n_), v->pool_[0][0].lastEle);

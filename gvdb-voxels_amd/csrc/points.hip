@@ -1272,7 +1272,7 @@ __device__ inline void k_push_gather_body(const BucketGatherArgs& a, uint32_t bi
     const int span = 2 + 2 * a.R, ncell = span * span * span;
     // (uniform) k_dense_gather's, by the record from which the host launches that one
     if (a.fullest > a.dense_cell && T > u64(a.dense_cell) * unsigned(ncell)) {
-        if (tid == 0) a.heavy[2 + atomicAdd(a.heavy, 1u)] = uint32_t(brick);
+        if (tid == 0) a.heavy[1 + atomicAdd(a.heavy, 1u)] = uint32_t(brick);
         return;
     }
     __syncthreads();                               // cell table and brick copy ready
@@ -1656,8 +1656,7 @@ __device__ inline void dense_brick(const BucketGatherArgs& a, int brick, DGShare
     __syncthreads();                               // the next brick may reuse S
 }
 
-// Workgroups of a grid take the listed bricks in turn; the last one to have
-// read the count clears it for the next launch.
+// Workgroups of a grid take the listed bricks in turn.
 template <typename AT>
 __global__ __launch_bounds__(DENSE_NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_dense_gather(BucketGatherArgs a0, MultiMap m) {
     __shared__ DGShared S;
@@ -1670,12 +1669,7 @@ __global__ __launch_bounds__(DENSE_NT) __attribute__((amdgpu_waves_per_eu(8, 8))
         bid -= m.first[g];
     }
     const uint32_t n = a->heavy[0];
-    __syncthreads();                               // all of the workgroup has read it
-    if (threadIdx.x == 0 && atomicAdd(a->heavy + 1, 1u) == nblk - 1) {
-        a->heavy[0] = 0;
-        a->heavy[1] = 0;
-    }
-    for (uint32_t i = bid; i < n; i += nblk) dense_brick<AT>(*a, int(a->heavy[2 + i]), S);
+    for (uint32_t i = bid; i < n; i += nblk) dense_brick<AT>(*a, int(a->heavy[1 + i]), S);
 }
 
 // The push gather's z slices per candidate, as the kernel computes it.
@@ -1707,17 +1701,24 @@ hipError_t launch_bucket_gather_multi(const BucketGatherArgs* a, int G, Arena* a
             nb.push_back(uint32_t(a[g].nleaves));
         }
         if (sel.empty()) continue;
+        // grids that can have dense bricks (the cells of a brick hold at most the
+        // fullest subcell's points each): their lists start empty
+        std::vector<FillArgs> empty;
+        if (kind < 4) {
+            for (const BucketGatherArgs& x : sel) {
+                if (!x.heavy) return hipErrorInvalidValue;
+                if (x.fullest > x.dense_cell) empty.push_back(FillArgs{x.heavy, 1, 0, 0});
+            }
+            const hipError_t e = launch_fill_multi(empty.data(), int(empty.size()), ar, s);
+            if (e != hipSuccess) return e;
+        }
         MultiLaunch L;
         // the push gather's multi-grid kernels read device tables only
         hipError_t e = multi_setup(ar, sel.data(), nb.data(), int(sel.size()), s, L, kind == 4);
         if (e != hipSuccess) return e;
         if (L.blocks == 0) continue;
         const dim3 grid(L.blocks);
-        if (kind < 4) {
-            for (const BucketGatherArgs& x : sel)
-                if (!x.heavy) return hipErrorInvalidValue;
-            L.map.xcd = knob(KNOB_XCD_ORDER);
-        }
+        if (kind < 4) L.map.xcd = knob(KNOB_XCD_ORDER);
         // the listed-slice variants run with the tuned threads per brick
         const bool wide = knob(KNOB_GATHER_THREADS) == 256;
         switch (variant) {
@@ -1746,14 +1747,9 @@ hipError_t launch_bucket_gather_multi(const BucketGatherArgs* a, int G, Arena* a
         }
         e = hipGetLastError();
         if (e != hipSuccess) return e;
-        if (kind == 4) continue;
-        // the dense bricks, the two workgroups a CU holds: for the grids that can
-        // have any (the cells of a brick hold at most the fullest subcell's
-        // points each)
-        size_t dense = 0;
-        for (const BucketGatherArgs& x : sel) dense += x.fullest > x.dense_cell ? 1 : 0;
-        if (!dense) continue;
-        const uint32_t each = std::max<uint32_t>(16u, 512u / uint32_t(dense));
+        // the dense bricks, the two workgroups a CU holds
+        if (empty.empty()) continue;
+        const uint32_t each = std::max<uint32_t>(16u, 512u / uint32_t(empty.size()));
         for (size_t g = 0; g < sel.size(); g++)
             nb[g] = sel[g].fullest > sel[g].dense_cell ? std::min(uint32_t(sel[g].nleaves), each) : 0;
         MultiLaunch D;

@@ -193,3 +193,24 @@ def test_eager_gather_after_a_replayed_insert(gpu, wait):
         assert np.array_equal(v.atlas().view(np.uint32), atlas["dense"])
     gr.close()
     v.close()
+
+
+def test_dense_bricks_after_a_refused_recording(gpu):
+    """A grid's first gather inside a recording grows its buffers, so the
+    recording is refused; the calls run directly afterwards all the same."""
+    pts, r = _points("full", 60000, 23), 2.0
+    want, _ = H.gpu_volume(gpu, pts, r)
+    v, n = H.gpu_volume(gpu, pts, r, stop_after="insert")
+    v.CaptureBegin()
+    v.GatherDensity(4, len(pts), r, H.ZERO3, n, 0, 0, False)
+    with pytest.raises(gpu.GVDBError) as e:
+        v.CaptureEnd()
+    assert e.value.code == gpu.ERR_STATE
+    for _ in range(2):
+        v.ClearChannel(0)
+        v.GatherDensity(4, len(pts), r, H.ZERO3, n, 0, 0, False)
+        v.UpdateApron(0, 0.0)
+        v.synchronize()
+        assert np.array_equal(v.atlas().view(np.uint32), want.atlas().view(np.uint32))
+    v.close()
+    want.close()
