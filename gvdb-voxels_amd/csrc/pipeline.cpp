@@ -1373,7 +1373,8 @@ int Volume::multi_render(Volume* const* vs, int G, const int* shading, const int
         a.t = v->make_tree();
         v->scene_block(r.w, r.h, a.s);
         a.tf = v->tf_dev.as<float4>();
-        a.tf_ramp = v->tf_ramp_ && v->tf_committed ? 1 : 0;
+        // (a recording keeps to the table, which later commits rewrite in place)
+        a.tf_ramp = v->tf_ramp_ && !ex.cap ? 1 : 0;
         for (int k = 0; k < 4; k++) { a.tf_a[k] = v->tf_a_[k]; a.tf_d[k] = v->tf_d_[k]; }
         a.atlas = v->chan_[c].data.p;
         a.out = r.data.p;

@@ -109,6 +109,43 @@ def test_graph_replay_one_grid(gpu):
     v.close()
 
 
+@pytest.mark.parametrize("side", [W, 400])     # four lanes a ray, one
+def test_recorded_render_takes_the_committed_transfer_function(gpu, side):
+    """A transfer function set and committed between replays is what the next
+    replay draws with, as the recorded march reads the device table; ramps over
+    the whole table and over a part of it."""
+    from gvdb_amd import workloads as Wk
+    c = (96.0, 96.0, 96.0)
+    pts = Wk.sphere_shell(20000, seed=43, radius=40.0, centre=c)
+    v = _grid(gpu, pts, c)
+    _chain(gpu, v, len(pts))
+    v.AddRenderBuf(0, side, side, 16)
+    sc = Wk.ea_scene(side, side, centre=c, dist=200.0)
+    tfs = [sc["tf"], (0.0, 1.0, (0.9, 0.1, 0.0, 0.2), (0.0, 0.7, 0.3, 1.0)),
+           (0.25, 0.75, (0.0, 0.0, 1.0, 0.5), (1.0, 1.0, 0.0, 0.9))]
+
+    def direct(tf):
+        v.apply_scene(dict(sc, tf=tf))
+        v.Render(gpu.SHADE_VOLUME, 0, 0)
+        return v.ReadRenderBuf(0, side, side, 16).view(np.uint32).copy()
+
+    direct(tfs[0])
+    v.CaptureBegin()
+    v.Render(gpu.SHADE_VOLUME, 0, 0)
+    g = v.CaptureEnd()
+    seen = []
+    for k in (1, 0, 2, 1):
+        v.apply_scene(dict(sc, tf=tfs[k]))
+        g.launch()
+        g.synchronize()
+        img = v.ReadRenderBuf(0, side, side, 16).view(np.uint32).copy()
+        assert np.array_equal(img, direct(tfs[k])), k
+        seen.append(img)
+    assert not np.array_equal(seen[0], seen[1]) and not np.array_equal(seen[1], seen[2])
+    g.close()
+    v.close()
+
+
 def test_calls_outside_the_chain_fail_the_recording(gpu):
     from gvdb_amd import workloads as Wk
     c = (64.0, 64.0, 64.0)
