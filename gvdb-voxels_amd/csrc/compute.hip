@@ -105,9 +105,8 @@ __device__ inline int layer_voxel(int f, int u, int w, int edge) {
 }
 
 // What the voxel beyond layer f of a slot comes from, in a.links[8 slot + f]:
-// the neighbour's slot (its layers), LINK_BOUND, or for a neighbour that the
-// operator does not reach -3 - slot (its voxels in the atlas).  LINK_OWN: the
-// slot holds no live brick, its apron stays as the atlas has it.
+// the neighbour's slot (its layers; below a.slots) or LINK_BOUND.  LINK_OWN:
+// the slot holds no live brick, its apron stays as the atlas has it.
 static const int LINK_BOUND = -1, LINK_OWN = -2;
 
 __device__ inline int link_of(const ComputeArgs& a, u64 slot, int f) {
@@ -117,9 +116,7 @@ __device__ inline int link_of(const ComputeArgs& a, u64 slot, int f) {
     if (base[13] != (long long)(slot * BRICK)) return LINK_OWN;
     const int step = f < 2 ? 1 : (f < 4 ? 3 : 9);
     const long long o = base[(f & 1) ? 13 + step : 13 - step];
-    if (o < 0) return LINK_BOUND;
-    const int ns = int(u64(o) / u64(BRICK));
-    return ns < a.slots ? ns : -3 - ns;
+    return o < 0 ? LINK_BOUND : int(u64(o) / u64(BRICK));
 }
 
 template <typename AT, bool FROM_CELLS, bool TO_CELLS>
@@ -155,8 +152,7 @@ __global__ __launch_bounds__(512) void k_compute_packed(ComputeArgs a) {
             const int q = wave * LAYERS + r, k = q / 6, f = q - k * 6;
             if (l[r] >= 0) g[r] = faces[u64(l[r]) * FACE_VALS + u64((f ^ 1) * 64 + lane)];
             else if (l[r] == LINK_BOUND) stv<AT>(&g[r], 0, a.boundval);
-            else if (l[r] == LINK_OWN) g[r] = atlas[(slot0 + k) * BRICK + layer_voxel(f, u, w, (f & 1) ? 9 : 0)];
-            else g[r] = atlas[u64(-3 - l[r]) * BRICK + layer_voxel(f, u, w, (f & 1) ? 1 : 8)];
+            else g[r] = atlas[(slot0 + k) * BRICK + layer_voxel(f, u, w, (f & 1) ? 9 : 0)];
         }
 #pragma unroll
         for (int k = 0; k < CB; k++)

@@ -201,6 +201,7 @@ int Volume::load_vbx(const char* path, int force_major, int force_minor) {
                 p.lastEle = p.usedNum = u64(cnt);
             }
         if (!fp.ok) return fail(GVDB_ERR_IO, "LoadVBX: truncated pools");
+        bool idle = false;   // a linked leaf is not in use
         // The kernels walk the pools without bounds checks, so every reference
         // a file holds must name a node or child list that exists: child list
         // ids, the child slots of each list, and parents.
@@ -232,12 +233,15 @@ int Volume::load_vbx(const char* path, int force_major, int force_minor) {
                 if (c != ID_UNDEF64 && ((c & 0xFF) != 0 || int((c >> 8) & 0xFF) != n - 1 ||
                                         (c >> 16) >= pool_[0][n - 1].lastEle))
                     return fail(GVDB_ERR_IO, "LoadVBX: child slot outside the pools");
+                if (n == 1 && c != ID_UNDEF64 && !reinterpret_cast<const Node*>(pool_[0][0].host.data())[c >> 16].mFlags)
+                    idle = true;
             }
         }
         if (root != ID_UNDEFL && ((root & 0xFF) != 0 || int((root >> 8) & 0xFF) >= levels ||
                                   (root >> 16) >= pool_[0][(root >> 8) & 0xFF].lastEle))
             return fail(GVDB_ERR_IO, "LoadVBX: root reference outside the pools");
         root_ = root;
+        loaded_idle_ = idle;
         host_valid_ = true;
         dev_stale_ = true;
         compute_top_lev();

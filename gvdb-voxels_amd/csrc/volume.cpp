@@ -451,6 +451,7 @@ int Volume::clear() {
         for (int l = 0; l < levels_; l++) { pool_[g][l].lastEle = 0; pool_[g][l].usedNum = 0; }
     root_ = ID_UNDEFL;
     atlas_used_ = 0;
+    loaded_idle_ = false;
     rebuild_topo_ = true;
     host_valid_ = true;
     dev_stale_ = false;
@@ -799,11 +800,14 @@ int Volume::compute(int effect, int c, int iterations, const float p[3], bool up
 
 // The smoothing's remaining `n` iterations with one apron at the end
 // (compute.hip); false where the neighbour table is not current (the first
-// iteration's apron builds it) or there is no room for the workspace, at most
-// LAYERS_MAX bytes, 840 k bricks in FP32 (then each iteration writes its apron).
+// iteration's apron builds it), where a brick's neighbour may have a slot past
+// the operator's (the layers are by slot), or where there is no room for the
+// workspace, at most LAYERS_MAX bytes, 840 k bricks in FP32 (then each
+// iteration writes its apron).
 bool Volume::smooth_layers(ComputeArgs a, int c, int n, float boundval, int& rc) {
     static const size_t LAYERS_MAX = size_t(4) << 30;
     if (brickwid_ != 8 || a.slots <= 0 || atlas_gen_ != topo_gen_ || nbr_gen_ != topo_gen_) return false;
+    if (loaded_idle_ || atlas_used_ > atlas_max_) return false;
     const size_t e = chan_[c].elem(), slots = size_t(a.slots);
     const size_t cells = slots * 512 * e, layer = slots * FACE_VALS * e, need = cells + 2 * layer + slots * 8 * sizeof(int);
     if (need > LAYERS_MAX) return false;

@@ -282,6 +282,7 @@ private:
     // The scatter gather's copy of each brick's boundary faces, current while
     // nothing else has written the atlas (atlas_epoch_ counts atlas writes).
     DevBuf faces_;
+    bool loaded_idle_ = false;   // a loaded file links leaves that are not in use, with atlas slots of their own
     DevBuf layers_;     // smoothing: interior voxels, two sets of boundary layers and their links, by slot
     DevBuf heavy_;      // bricks the scatter gather leaves to the dense one (BucketGatherArgs::heavy)
     unsigned atlas_epoch_ = 0, faces_epoch_ = ~0u, faces_topo_ = ~0u;

@@ -35,3 +35,24 @@ def test_iterations_in_one_call_equal_single_calls(gpu, effect, params, half, bo
         v.close()
     a, b = (x.view(np.uint16 if half else np.uint32) for x in out)
     assert np.array_equal(a, b), "%d voxels differ" % int((a != b).sum())
+
+
+def test_channel_created_again_smaller(gpu):
+    """Channel 0 created again with fewer slots than the bricks had: the
+    operator takes the slots there are; their neighbours lie past them."""
+    from gvdb_amd import workloads as W
+    pts = W.sphere_shell(3000, seed=17, radius=40.0, centre=(64.0, 64.0, 64.0))
+    out = []
+    for calls in ((3,), (1, 1, 1)):
+        v, _ = H.gpu_volume(gpu, pts, 2.0, axiscnt=(16, 16, 8))
+        used = v.atlas_info()["used"]
+        assert 16 * 16 < used <= 16 * 16 * 8
+        v.SetChannelDefault(16, 16, 1)
+        v.AddChannel(0, gpu.T_FLOAT, 1)
+        v.Compute(gpu.FUNC_FILL_F, 0, 1, (1.0, 0.0, 0.0), False, False, 0.0)
+        for n in calls:
+            v.Compute(gpu.FUNC_SMOOTH, 0, n, (2.0, 0.0, 0.0), True, True, 0.5)
+        v.synchronize()
+        out.append(v.atlas().view(np.uint32).copy())
+        v.close()
+    assert np.array_equal(out[0], out[1])

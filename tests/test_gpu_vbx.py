@@ -190,3 +190,40 @@ def test_load_vbx_errors(gpu, tmp_path):
     w.LoadVBX(write("same.vbx", p0, p1))
     v.close()
     w.close()
+
+
+def test_smoothing_beside_an_idle_leaf_of_a_file(gpu, tmp_path):
+    """A file may link a leaf that is not in use, whose atlas slot is its own and
+    may lie past those of the used ones; the aprons beside it hold its voxels.
+    Several smoothing passes in one call equal single ones there too."""
+    import vbx
+    from gvdb_amd import workloads as W
+    pts = W.sphere_shell(3000, seed=83, radius=20.0, centre=(64.0, 64.0, 64.0))
+    v, _ = H.gpu_volume(gpu, pts, 2.0, axiscnt=(16, 16, 3))
+    p0 = [v.pool(0, l).copy() for l in range(5)]
+    p1 = [v.pool(1, l).copy() if l else None for l in range(5)]
+    pos = p0[0]["mPos"]
+    near = (np.abs(pos[:, None, :] - pos[None]).sum(-1) == 8).sum(1)      # face neighbours
+    idle = int(np.argmax(near))
+    assert near[idle] >= 3 and len(pos) < 16 * 16 * 3 - 40
+    atlas = v.atlas().copy()
+    x, y, z = p0[0]["mValue"][idle] - 1
+    cx, cy, cz = 150, 140, 20                                             # slot (15, 14, 2)
+    atlas[cz:cz + 10, cy:cy + 10, cx:cx + 10] = atlas[z:z + 10, y:y + 10, x:x + 10] + np.float32(0.25)
+    p0[0]["mFlags"][idle] = 0
+    p0[0]["mValue"][idle] = (cx + 1, cy + 1, cz + 1)
+    (tmp_path / "idle.vbx").write_bytes(vbx.write_vbx(_meta(v), [q.tobytes() for q in p0],
+                                                      [q.tobytes() if q is not None else b"" for q in p1], [(3, atlas)]))
+    v.close()
+    out = []
+    for calls in ((4,), (1, 1, 1, 1)):
+        w = gpu.VolumeGVDB(0)
+        w.LoadVBX(str(tmp_path / "idle.vbx"))
+        for n in calls:
+            w.Compute(gpu.FUNC_SMOOTH, 0, n, (2.0, 0.0, 0.0), True, True, 0.5)
+        w.synchronize()
+        a = w.atlas()
+        assert np.array_equal(a[cz + 1:cz + 9, cy + 1:cy + 9, cx + 1:cx + 9], atlas[cz + 1:cz + 9, cy + 1:cy + 9, cx + 1:cx + 9])
+        out.append(a.view(np.uint32))
+        w.close()
+    assert np.array_equal(out[0], out[1])
