@@ -1185,8 +1185,9 @@ int Volume::multi_gather(Volume* const* vs, int G, int scs, const int* len, cons
         v->atlas_epoch_++;
         if (buckets) {
             // the scatter kernel (no accumulate) also leaves the bricks' faces for the apron
+            // (not those of leaves out of use, whose voxels only the atlas has)
             void* faces = nullptr;
-            if (!accum && !levelset) {
+            if (!accum && !levelset && !v->loaded_idle_) {
                 const size_t need = size_t(v->pool_[0][0].lastEle) * FACE_VALS * v->chan_[chanD].elem();
                 if (v->faces_.ensure(need) == hipSuccess) {
                     faces = v->faces_.p;

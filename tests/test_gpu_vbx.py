@@ -192,10 +192,10 @@ def test_load_vbx_errors(gpu, tmp_path):
     w.close()
 
 
-def test_smoothing_beside_an_idle_leaf_of_a_file(gpu, tmp_path):
-    """A file may link a leaf that is not in use, whose atlas slot is its own and
-    may lie past those of the used ones; the aprons beside it hold its voxels.
-    Several smoothing passes in one call equal single ones there too."""
+def _idle_leaf_file(gpu, path):
+    """Writes a grid in which a leaf with neighbours is linked but not in use,
+    its voxels in a slot past those of the used leaves; returns the points, the
+    slot's first voxel (x, y, z) and the atlas."""
     import vbx
     from gvdb_amd import workloads as W
     pts = W.sphere_shell(3000, seed=83, radius=20.0, centre=(64.0, 64.0, 64.0))
@@ -212,9 +212,16 @@ def test_smoothing_beside_an_idle_leaf_of_a_file(gpu, tmp_path):
     atlas[cz:cz + 10, cy:cy + 10, cx:cx + 10] = atlas[z:z + 10, y:y + 10, x:x + 10] + np.float32(0.25)
     p0[0]["mFlags"][idle] = 0
     p0[0]["mValue"][idle] = (cx + 1, cy + 1, cz + 1)
-    (tmp_path / "idle.vbx").write_bytes(vbx.write_vbx(_meta(v), [q.tobytes() for q in p0],
-                                                      [q.tobytes() if q is not None else b"" for q in p1], [(3, atlas)]))
+    path.write_bytes(vbx.write_vbx(_meta(v), [q.tobytes() for q in p0], [q.tobytes() if q is not None else b"" for q in p1],
+                                   [(3, atlas)]))
     v.close()
+    return pts, (cx, cy, cz), atlas
+
+
+def test_smoothing_beside_an_idle_leaf_of_a_file(gpu, tmp_path):
+    """The aprons beside a linked leaf that is not in use hold its voxels.
+    Several smoothing passes in one call equal single ones there too."""
+    _, (cx, cy, cz), atlas = _idle_leaf_file(gpu, tmp_path / "idle.vbx")
     out = []
     for calls in ((4,), (1, 1, 1, 1)):
         w = gpu.VolumeGVDB(0)
@@ -223,7 +230,26 @@ def test_smoothing_beside_an_idle_leaf_of_a_file(gpu, tmp_path):
             w.Compute(gpu.FUNC_SMOOTH, 0, n, (2.0, 0.0, 0.0), True, True, 0.5)
         w.synchronize()
         a = w.atlas()
-        assert np.array_equal(a[cz + 1:cz + 9, cy + 1:cy + 9, cx + 1:cx + 9], atlas[cz + 1:cz + 9, cy + 1:cy + 9, cx + 1:cx + 9])
+        box = (slice(cz + 1, cz + 9), slice(cy + 1, cy + 9), slice(cx + 1, cx + 9))
+        assert np.array_equal(a[box], atlas[box])
         out.append(a.view(np.uint32))
         w.close()
     assert np.array_equal(out[0], out[1])
+
+
+def test_aprons_beside_an_idle_leaf_after_a_gather(gpu, tmp_path):
+    """UpdateApron right after GatherDensity gives what it gives after another
+    call has written the atlas (noise of amplitude 0)."""
+    pts, _, _ = _idle_leaf_file(gpu, tmp_path / "idle.vbx")
+    w = gpu.VolumeGVDB(0)
+    w.LoadVBX(str(tmp_path / "idle.vbx"))
+    w.SetPoints(pts)
+    n = w.InsertPointsSubcell(4, len(pts), 2.0, H.ZERO3)
+    w.GatherDensity(4, len(pts), 2.0, H.ZERO3, n, 0, 0, False)
+    w.UpdateApron(0, 0.0)
+    w.synchronize()
+    a = w.atlas().view(np.uint32).copy()
+    w.Compute(gpu.FUNC_NOISE, 0, 1, (0.0, 0.0, 0.0), True, True, 0.0)
+    w.synchronize()
+    assert np.array_equal(w.atlas().view(np.uint32), a)
+    w.close()
