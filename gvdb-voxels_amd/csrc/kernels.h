@@ -530,6 +530,9 @@ struct RenderArgs {
     const uint32_t* clr; // the colour channel (uchar4 per voxel, SetColorChannel), or null
 };
 hipError_t launch_render_multi(const RenderArgs* a, int G, Arena* ar, hipStream_t s);
+// Does the call's march of the first image's mode depend on the launch-shape
+// knobs (KNOB_RENDER_*)?  Reads t, the image sizes, shading and atlas_type.
+bool render_reads_knobs(const RenderArgs* a, int G);
 
 // ---- launch-shape knobs (tune.cpp), process-wide, picked by the autotuner
 enum Knob {

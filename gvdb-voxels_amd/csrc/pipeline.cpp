@@ -1345,6 +1345,20 @@ int Volume::update_apron_noalloc(int c, float boundval) {
 }
 
 // ---------------------------------------------------------------- Render ----
+bool Volume::multi_render_reads_knobs(Volume* const* vs, int G, const int* shading, const int* chan, const int* buf) {
+    std::vector<RenderArgs> ra(G);
+    for (int g = 0; g < G; g++) {
+        Volume* v = vs[g];
+        if (buf[g] < 0 || buf[g] >= 4 || chan[g] < 0 || chan[g] >= 8) return true;
+        ra[g].t = v->make_tree();
+        ra[g].s.width = v->rbuf_[buf[g]].w;
+        ra[g].s.height = v->rbuf_[buf[g]].h;
+        ra[g].shading = shading[g];
+        ra[g].atlas_type = v->chan_[chan[g]].type;
+    }
+    return gvdb::render_reads_knobs(ra.data(), G);
+}
+
 int Volume::multi_render(Volume* const* vs, int G, const int* shading, const int* chan, const int* buf, const Exec& ex,
                          int* failed) {
     // Render (gvdb_volume_gvdb.cpp:4336-4381)

@@ -785,21 +785,35 @@ static float pow2_inverse(float d) {
     return std::fabs(m) == 0.5f && e > -100 && e < 100 ? 1.0f / d : 0.0f;
 }
 
+// One launch per variant of the kernel: bit 0 isosurface, 1 half, 2 not ten_sided.
+static int variant_of(const RenderArgs& a) {
+    return (a.shading == SHADE_VOLUME ? 0 : 1) | (a.atlas_type == T_HALF ? 2 : 0) | (ten_sided(a.t) ? 0 : 4);
+}
+// Do the images of `variant` (if any) go with four lanes per ray?
+static bool split_of(const RenderArgs* a, int G, int variant) {
+    u64 rays = 0;
+    for (int g = 0; g < G; g++)
+        if (variant_of(a[g]) == variant) rays += u64(a[g].s.width) * u64(a[g].s.height);
+    return !(variant & 4) && rays <= SPLIT_RAYS;
+}
+
+bool render_reads_knobs(const RenderArgs* a, int G) {
+    for (int g = 0; g < G; g++)
+        if (variant_of(a[g]) % 2 == variant_of(a[0]) % 2 && !split_of(a, G, variant_of(a[g]))) return true;
+    return false;
+}
+
 hipError_t launch_render_multi(const RenderArgs* a, int G, Arena* ar, hipStream_t s) {
+    for (int g = 0; g < G; g++)
+        if (a[g].shading != SHADE_VOLUME && a[g].shading != SHADE_TRILINEAR) return hipErrorInvalidValue;
     for (int variant = 0; variant < 8; variant++) {
         const int mode = variant & 1;
         const bool half = variant & 2, ten = !(variant & 4);
         std::vector<RenderArgs> sel;
-        u64 rays = 0;
-        for (int g = 0; g < G; g++) {
-            if (a[g].shading != SHADE_VOLUME && a[g].shading != SHADE_TRILINEAR) return hipErrorInvalidValue;
-            const int am = a[g].shading == SHADE_VOLUME ? 0 : 1;
-            if (am != mode || (a[g].atlas_type == T_HALF) != half || ten_sided(a[g].t) != ten) continue;
-            sel.push_back(a[g]);
-            rays += u64(a[g].s.width) * u64(a[g].s.height);
-        }
+        for (int g = 0; g < G; g++)
+            if (variant_of(a[g]) == variant) sel.push_back(a[g]);
         if (sel.empty()) continue;
-        const bool split = ten && rays <= SPLIT_RAYS;
+        const bool split = split_of(sel.data(), int(sel.size()), variant);
         const int per = split ? 64 / SPLIT : 64;
         const int tw = split ? 4 : knob(mode ? KNOB_RENDER_TILE_ISO : KNOB_RENDER_TILE_EA), th = per / tw;
         std::vector<uint32_t> nb;

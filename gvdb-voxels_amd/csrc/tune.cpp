@@ -60,9 +60,12 @@ static int time_runs(F&& run, float& out) {
 
 // Tries every value of the knobs in `ks` (all combinations), keeps the
 // fastest; ms[] gets one time per combination, the first knob varying
-// slowest.  On failure the knobs are restored.
+// slowest.  On failure the knobs are restored.  A call that does not read the
+// knobs (reads = false) is timed once, its time stands for every combination
+// and the knobs stay: picking the least of equal launches would set them for
+// every later launch by chance.
 template <class F>
-static int tune_knobs(const int* ks, int nk, F&& run, int* best, float* ms) {
+static int tune_knobs(const int* ks, int nk, F&& run, int* best, float* ms, bool reads = true) {
     int vals[2][KNOB_MAX_VALUES], cnt[2] = {1, 1}, keep[2] = {0, 0};
     for (int i = 0; i < nk; i++) {
         cnt[i] = knob_values(ks[i], vals[i]);
@@ -71,6 +74,14 @@ static int tune_knobs(const int* ks, int nk, F&& run, int* best, float* ms) {
     float best_ms = FLT_MAX;
     int pick[2] = {keep[0], keep[1]};
     int idx = 0;
+    if (!reads) {
+        float t = 0.f;
+        int rc = time_runs(run, t);
+        if (rc != GVDB_OK) return rc;
+        for (int i = 0; ms && i < cnt[0] * cnt[1]; i++) ms[i] = t;
+        for (int i = 0; best && i < nk; i++) best[i] = keep[i];
+        return GVDB_OK;
+    }
     for (int a = 0; a < cnt[0]; a++)
         for (int b = 0; b < (nk > 1 ? cnt[1] : 1); b++, idx++) {
             g_knob[ks[0]] = vals[0][a];
@@ -106,7 +117,7 @@ int tune_render(Volume& v, int shading, int chan, int buf, int* best2, float* ms
         if (r == GVDB_OK) r = v.kernel_ms(k);
         ms = k[2];
         return r;
-    }, b, ms12);
+    }, b, ms12, v.render_reads_knobs(shading, chan, buf));
     if (rc == GVDB_OK && best2) {
         best2[0] = b[1];   // unroll
         best2[1] = b[0];   // tile width
@@ -123,7 +134,7 @@ int tune_render_unroll(Volume& v, int shading, int chan, int buf, int* best, flo
         if (r == GVDB_OK) r = v.kernel_ms(k);
         ms = k[2];
         return r;
-    }, best, ms3);
+    }, best, ms3, v.render_reads_knobs(shading, chan, buf));
 }
 
 int tune_gather(Volume& v, int scs, int n, float radius, const float trans[3], int len, int chan, int* best,
@@ -193,7 +204,8 @@ int tune_batch(Batch& B, Volume* const* vs, int G, int stage, int scs, const int
         const int ks[2] = {ea ? KNOB_RENDER_TILE_EA : KNOB_RENDER_TILE_ISO,
                            ea ? KNOB_RENDER_UNROLL_EA : KNOB_RENDER_UNROLL_ISO};
         int b[2];
-        int rc = tune_knobs(ks, 2, timed([&] { return B.render(vs, G, shading, chans, bufs, failed); }), b, ms);
+        int rc = tune_knobs(ks, 2, timed([&] { return B.render(vs, G, shading, chans, bufs, failed); }), b, ms,
+                            Volume::multi_render_reads_knobs(vs, G, shading, chans, bufs));
         if (rc == GVDB_OK && best) {
             best[0] = b[1];
             best[1] = b[0];

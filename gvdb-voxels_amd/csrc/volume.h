@@ -226,6 +226,12 @@ public:
                            const void* slot_faces = nullptr);
     static int multi_render(Volume* const* v, int G, const int* shading, const int* chan, const int* buf, const Exec& ex,
                             int* failed);
+    // does this render depend on the launch-shape knobs (true for arguments the render refuses)
+    static bool multi_render_reads_knobs(Volume* const* v, int G, const int* shading, const int* chan, const int* buf);
+    bool render_reads_knobs(int shading, int chan, int buf) {
+        Volume* v = this;
+        return multi_render_reads_knobs(&v, 1, &shading, &chan, &buf);
+    }
     int hip_fail(hipError_t e, const char* what);
 
 private:

@@ -212,7 +212,9 @@ int gvdb_read_render_buf(gvdb_handle h, int buf, void* host_dst);
 /* Autotuner (no counterpart in the reference; for callers that run one workload shape many times).  The launch-shape
  * knobs below change no result, only time; each tuner runs the caller's own workload once per value (a warm-up, then
  * the median of three runs timed with HIP events on the handle's or batch's stream) and keeps the fastest,
- * process-wide.  Times go to ms[] in the order of the knob's values (may be NULL). */
+ * process-wide.  Times go to ms[] in the order of the knob's values (may be NULL).  A render of up to 98,304 rays in
+ * all (8^3 bricks, apron 1) takes four lanes per ray and reads neither render knob: its tuners time it once, give that
+ * time for every value and leave the knobs as they are. */
 #define GVDB_KNOB_RENDER_UNROLL_EA 0  /* samples fetched ahead per brick step, SHADE_VOLUME: 1, 2, 4 */
 #define GVDB_KNOB_RENDER_UNROLL_ISO 1 /* the same, SHADE_TRILINEAR */
 #define GVDB_KNOB_RENDER_TILE_EA 2    /* ray-packet width of a 64-lane workgroup (8x8, 16x4, 32x2, 64x1): 8..64 */

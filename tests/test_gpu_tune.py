@@ -63,6 +63,36 @@ def test_render_every_packet_shape_and_unroll_same_pixels(gpu, restore_knobs, sh
     v.close()
 
 
+def test_small_render_leaves_the_knobs(gpu, restore_knobs):
+    """A launch of few rays takes four lanes per ray and no knob: its tuners
+    (both forms, and a batch's) give one time for all values and keep them; a
+    larger image's choose."""
+    from gvdb_amd import workloads as W
+    pts = W.sphere_shell(20000, seed=24, radius=40.0, centre=(64.0, 64.0, 64.0))
+    v, _ = _grid(gpu, pts)
+    mode, kt, ku = gpu.SHADE_VOLUME, gpu.KNOB_RENDER_TILE_EA, gpu.KNOB_RENDER_UNROLL_EA
+    w = 256
+    v.apply_scene(W.ea_scene(w, w, centre=(64.0, 64.0, 64.0), dist=200.0))
+    v.AddRenderBuf(0, w, w, 16)
+    B = gpu.GridBatch(0, 1)
+    for tw, u in ((32, 1), (64, 2), (16, 4)):
+        gpu.set_tuning(kt, tw)
+        gpu.set_tuning(ku, u)
+        for best, ms in (v.TuneRenderShape(mode), B.Tune([v], "render", shading=mode)):
+            assert tuple(best) == (u, tw) and len(set(ms.values())) == 1 and min(ms.values()) > 0
+        best, ms = v.TuneRender(mode)
+        assert best == u and len(set(ms.values())) == 1
+        assert gpu.get_tuning(kt)[0] == tw and gpu.get_tuning(ku)[0] == u
+    # 98,304 rays: the last such image; one row more and the tuner measures
+    v.AddRenderBuf(1, 256, 384, 16)
+    v.AddRenderBuf(2, 256, 385, 16)
+    assert len(set(v.TuneRenderShape(mode, 0, 1)[1].values())) == 1
+    best, ms = v.TuneRenderShape(mode, 0, 2)
+    assert len(set(ms.values())) > 1 and ms[(best[1], best[0])] == min(ms.values())
+    B.close()
+    v.close()
+
+
 @pytest.mark.parametrize("radius", [2.0, 2.25])
 def test_gather_threads_same_atlas(gpu, restore_knobs, radius):
     from gvdb_amd import workloads as W
