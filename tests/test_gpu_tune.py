@@ -63,6 +63,51 @@ def test_render_every_packet_shape_and_unroll_same_pixels(gpu, restore_knobs, sh
     v.close()
 
 
+@pytest.mark.parametrize("shading", ["volume", "trilinear"])
+@pytest.mark.parametrize("dims,half", [((3, 3, 3, 4, 5), False), ((3, 3, 3, 4, 5), True), ((2, 3, 3, 4, 5), False),
+                                       ((2, 3, 3, 4, 5), True)])
+def test_knobs_same_pixels_past_the_small_render_line(gpu, restore_knobs, shading, dims, half):
+    """Every ray-packet shape and number of samples ahead where the launch reads
+    them (more rays than take four lanes each): the same pixels on 8^3 and 4^3
+    bricks, float and half."""
+    from gvdb_amd import workloads as W
+    pts = W.sphere_shell(20000, seed=25, radius=40.0, centre=(64.0, 64.0, 64.0))
+    v = gpu.VolumeGVDB(0)
+    v.Configure(*reversed(dims))
+    v.SetChannelDefault(16, 16, 4)
+    v.AddChannel(0, gpu.T_HALF if half else gpu.T_FLOAT, 1)
+    v.SetPoints(pts)
+    v.RequestFullRebuild(True)
+    v.RebuildTopology(len(pts), 2.0, H.ZERO3)
+    v.FinishTopology(False, True)
+    v.UpdateAtlas()
+    v.ClearChannel(0)
+    n = v.InsertPointsSubcell(4, len(pts), 2.0, H.ZERO3)
+    v.GatherDensity(4, len(pts), 2.0, H.ZERO3, n, 0, 0, False)
+    v.UpdateApron(0, 0.0)
+    w, h = 331, 303     # partial tiles of every shape
+    if shading == "volume":
+        sc, mode = W.ea_scene(w, h, centre=(64.0, 64.0, 64.0), dist=200.0), gpu.SHADE_VOLUME
+        kt, ku = gpu.KNOB_RENDER_TILE_EA, gpu.KNOB_RENDER_UNROLL_EA
+    else:
+        sc, mode = W.iso_scene(w, h, centre=(64.0, 64.0, 64.0), dist=200.0), gpu.SHADE_TRILINEAR
+        kt, ku = gpu.KNOB_RENDER_TILE_ISO, gpu.KNOB_RENDER_UNROLL_ISO
+    v.apply_scene(sc)
+    v.AddRenderBuf(0, w, h, 16)
+    ref = None
+    for tw in (8, 16, 32, 64):
+        for u in (1, 2, 4):
+            gpu.set_tuning(kt, tw)
+            gpu.set_tuning(ku, u)
+            v.Render(mode, 0, 0)
+            img = v.ReadRenderBuf(0, w, h, 16)
+            if ref is None:
+                ref = img.copy()
+                assert np.count_nonzero(np.abs(img - np.asarray(sc["backclr"], np.float32)).max(-1)) > 1000
+            assert np.array_equal(img.view(np.uint32), ref.view(np.uint32)), (tw, u)
+    v.close()
+
+
 def test_small_render_leaves_the_knobs(gpu, restore_knobs):
     """A launch of few rays takes four lanes per ray and no knob: its tuners
     (both forms, and a batch's) give one time for all values and keep them; a
