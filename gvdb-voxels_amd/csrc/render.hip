@@ -106,7 +106,8 @@ __device__ inline void tri_fetch(const AT* b, int br_rt, const Corner& K, float 
     unsigned at;
     if constexpr (BR != 0) {
         const float f = __builtin_fmaf(fz0, float(BR * BR), __builtin_fmaf(fy0, float(BR), fx0 - K.base));
-        at = min(unsigned(f), unsigned((BR - 2) * (BR * BR + BR + 1)));
+        // (f < 0 or past the brick: a sample past a face, fetched but never used)
+        at = unsigned(__builtin_amdgcn_fmed3f(f, 0.0f, float((BR - 2) * (BR * BR + BR + 1))));
     } else {
         const int ix = min(max(int(fx0) - K.c[0], 0), br - 2), iy = min(max(int(fy0) - K.c[1], 0), br - 2),
                   iz = min(max(int(fz0) - K.c[2], 0), br - 2);
