@@ -96,9 +96,18 @@ struct MarkArgs {
 // pack: byte marks go on to the bitmaps (otherwise launch_box_levels_multi reads them)
 hipError_t launch_mark_points_multi(const MarkArgs* a, int G, Arena* ar, hipStream_t s, bool pack);
 
-// Byte marks to every level's bitmaps, ranks and counts in one workgroup, for
-// boxes whose bitmaps take at most BOX_WORDS words in all.
-static const uint32_t BOX_WORDS = 15360;
+// Byte marks to every level's bitmaps, ranks and counts in one workgroup per
+// grid, for boxes whose bitmaps take at most box_words(grids) words in all.
+// The line: a large box holds one CU while the launches level by level spread
+// over all of them; those are several short ones, whose fixed times many grids
+// share.  Measured, us, this way / level by level, by words of level 0.  One
+// grid's rebuild: 580 70.4 / 71.7, 1862 73.0 / 72.5, 4308 84.4 / 78.4, 7688
+// 115.5 / 99.9; a whole splat, alone: 1862 322 / 324, 2916 334 / 335, 4308 347 /
+// 343, 8292 387 / 373; among others on other streams: 256 254 / 261, 2784 590 /
+// 600, 2916 278 / 277, 4308 290 / 286.  Rebuild of 4 grids: 4000 93.1 / 93.5,
+// 6490 105.5 / 99.4; of 16: 4000 145 / 167, 10400 199 / 212.
+static const uint32_t BOX_WORDS = 15360;   // what the workgroup's LDS holds
+inline u64 box_words(int grids) { return 3072 + 512 * u64(grids - 1) < BOX_WORDS ? 3072 + 512 * u64(grids - 1) : BOX_WORDS; }
 static const int BOX_LEVELS = 5;
 struct BoxArgs {
     const uint8_t* bytes;

@@ -315,7 +315,7 @@ int Volume::multi_full_build(Volume* const* vs, int G, const int* n, const float
             pl.masks = v->masks_.as<uint32_t>();
             fills.push_back(FillArgs{pl.masks, pl.dom[0].nbits, 0, 0});
         }
-        boxed = boxed && path == 1 && pl.bm_words <= BOX_WORDS && D <= BOX_LEVELS;
+        boxed = boxed && path == 1 && pl.bm_words <= box_words(G) && D <= BOX_LEVELS;
     }
     if (!boxed)
         for (int g = 0; g < G; g++) fills.push_back(FillArgs{vs[g]->bitmaps_.p, plan[g].bm_words, 0, 0});

@@ -49,12 +49,41 @@ def _box(side, n, seed, lo=(0.0, 0.0, 0.0)):
     return p.astype(np.float32)
 
 
-# 15360 words of bitmaps in all: with dilation about 245,000 bricks, 62 a side
-# (496 voxels); without, 491,000 (78 a side)
+# small boxes (one workgroup) and large ones (level by level), up to four levels
 @pytest.mark.parametrize("r,side", [(2.0, (40, 20, 40)), (2.0, (480, 480, 480)), (2.0, (505, 500, 498)), (0.5, (500, 500, 500)),
                                     (0.5, (640, 640, 640)), (5.5, (70, 400, 33)), (2.0, (3000, 40, 40)), (1.0, (9, 9, 9))])
 def test_levels_and_bounds(gpu, r, side):
     _check(gpu, _box(side, 3000, 5, (17.5, 33.0, 72.25)), r)
+
+
+# one grid takes the one-workgroup form up to 3072 words (49,000 bricks with
+# dilation, 36 a side), each further one of a batch adds 512
+@pytest.mark.parametrize("side", [(262, 260, 262), (272, 270, 273), (277, 278, 276), (282, 283, 281), (300, 300, 300)])
+def test_levels_around_the_one_grid_limit(gpu, side):
+    _check(gpu, _box(side, 3000, 6, (17.5, 33.0, 72.25)), 2.0)
+
+
+@pytest.mark.parametrize("grids,side", [(2, 285), (2, 305), (5, 320), (5, 345), (30, 470), (30, 510)])
+def test_levels_of_a_batch_around_its_limit(gpu, grids, side):
+    """The largest grid decides for the call; pools equal those of single calls."""
+    sets = [_box((side, side, side) if k == 1 else (40 + 9 * k, 50, 60), 800, 7 + k, (17.5, 33.0, 72.25)) for k in range(grids)]
+    vols = []
+    for p in sets:
+        v = gpu.VolumeGVDB(0)
+        v.Configure(*H.TREE)
+        v.SetPoints(p)
+        v.RequestFullRebuild(True)
+        vols.append(v)
+    b = gpu.GridBatch(0, grids)
+    b.RebuildTopology(vols, [len(p) for p in sets], 2.0)
+    b.synchronize()
+    for v, p in zip(vols, sets):
+        one, _ = H.gpu_volume(gpu, p, 2.0, stop_after="topology")
+        H.assert_pools_equal(v, one)
+        one.close()
+    b.close()
+    for v in vols:
+        v.close()
 
 
 def test_bounds_at_the_root_corner_and_border(gpu):
