@@ -301,6 +301,7 @@ int Volume::add_channel(int c, int dtype, int apron, int filter, int border, int
     ch.border = border;
     int br = brickwid_ + 2 * apron_;
     size_t bytes = size_t(atlas_max_) * br * br * br * ch.elem();
+    if (bytes > ch.data.bytes) layers_.release();   // as when the atlas grows
     HIPCHK(ch.data.ensure(bytes));
     HIPCHK(launch_fill_u32(ch.data.as<uint32_t>(), 0u, ch.data.bytes / 4, stream));
     return GVDB_OK;
@@ -644,6 +645,7 @@ int Volume::resize_atlas(int cz) {
         size_t old = size_t(atlas_max_) * br * br * br * ch.elem();
         size_t need = size_t(slots) * br * br * br * ch.elem();
         if (need > ch.data.bytes) {
+            layers_.release();   // sized for the old atlas; the next smoothing makes its own
             DevBuf nb;
             HIPCHK(nb.ensure(need));
             HIPCHK(launch_fill_u32(nb.as<uint32_t>(), 0u, nb.bytes / 4, stream));

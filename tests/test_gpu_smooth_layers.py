@@ -56,3 +56,42 @@ def test_channel_created_again_smaller(gpu):
         out.append(v.atlas().view(np.uint32).copy())
         v.close()
     assert np.array_equal(out[0], out[1])
+
+
+def _free_bytes(gpu):
+    """Free device memory by the HIP runtime the library is linked to."""
+    import ctypes
+    gpu.load()
+    with open("/proc/self/maps") as f:
+        libs = sorted({x.split()[-1] for x in f if "libamdhip64" in x}, key=lambda x: "/opt/rocm" not in x)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL(libs[0]).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_workspace_goes_back_when_the_atlas_grows(gpu):
+    """A grid that has smoothed holds no more memory than one that has not,
+    once its atlas had to grow (the workspace is the size of the old atlas)."""
+    from gvdb_amd import workloads as W
+    small, large = W.sphere_shell(120000, seed=18), W.sphere_shell(300000, seed=19, radius=170.0)
+    used, held = {}, 0
+    for smooth in (False, True, False, True):
+        f0 = _free_bytes(gpu)
+        v, _ = H.gpu_volume(gpu, small, 2.0)
+        f1 = _free_bytes(gpu)
+        if smooth:
+            v.Compute(gpu.FUNC_SMOOTH, 0, 4, (2.0, 0.0, 0.0), True, True, 0.0)
+            v.synchronize()
+            held = f1 - _free_bytes(gpu)
+        slots = v.atlas_info()["cnt"][2]
+        v.SetPoints(large)
+        v.RequestFullRebuild(True)
+        v.RebuildTopology(len(large), 2.0, H.ZERO3)
+        v.FinishTopology(False, True)
+        v.UpdateAtlas()
+        v.synchronize()
+        assert v.atlas_info()["cnt"][2] > slots
+        used[smooth] = f0 - _free_bytes(gpu)
+        v.close()
+    assert held > 20 << 20
+    assert used[True] - used[False] < held / 4, (used, held)
