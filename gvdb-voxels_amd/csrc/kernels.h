@@ -551,7 +551,7 @@ enum Knob {
     KNOB_RENDER_TILE_ISO,
     KNOB_GATHER_THREADS,         // threads per brick of the scatter gather at radius <= 3: 128, 256
     KNOB_APRON_RUN,              // bricks per workgroup of the multi-grid apron: 1, 2, 4, 8
-    KNOB_XCD_ORDER,              // per-brick kernels: 0 launch order, 1 each XCD a contiguous range of bricks
+    KNOB_XCD_ORDER,              // per-brick kernels: 0 launch order, 1 each XCD a contiguous range of bricks (always 1 for aprons that read whole bricks)
     KNOB_APRON_QUEUE,            // multi-grid apron: 0 static runs, 1 persistent workgroups over a brick queue
     KNOB_MARK_PATH,              // topology marks: 0 by domain size, 1 a byte per brick, 2 direction masks, 3 bits,
                                  // 4 sorted brick keys (the build taken above 2^34 bricks)

@@ -581,7 +581,7 @@ hipError_t launch_leaf_bounds_multi(const BoundsArgs* a, int G, Arena* ar, hipSt
 // neighbourhood fits in the 27 bricks around; otherwise the push kernels run.
 namespace gvdb {
 
-static const int LEN_PARTS = 64;   // spread counters of the entry count; as many words with the largest slot follow
+static const int LEN_PARTS = 64;   // spread counters of the entry count; as many flags (BucketArgs::len) follow
 
 __device__ inline void k_bucket_points_body(const BucketArgs& a, uint32_t bid, uint32_t) {
     const Tree& t = a.t;
@@ -683,9 +683,9 @@ __device__ inline void k_bucket_points_body(const BucketArgs& a, uint32_t bid, u
     }
 }
 
-// Sum of a grid's LEN_PARTS entry counters into its result word.
-// (and the orphan count beside it: both go to host memory when the host is the
-// only reader)
+// Sum of a grid's LEN_PARTS entry counters into its result word, whether any
+// flag is set, and the orphan count (to host memory when the host is the only
+// reader).
 __device__ inline void k_sum_parts_body(const SumArgs& a, uint32_t, uint32_t) {
     u64 v = threadIdx.x < LEN_PARTS ? a.parts[threadIdx.x] : 0ull;
     uint32_t f = reinterpret_cast<const uint32_t*>(a.parts + LEN_PARTS)[threadIdx.x];

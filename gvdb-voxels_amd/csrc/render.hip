@@ -12,9 +12,11 @@
 // four lanes per ray when a launch has few rays).
 //
 // What bounds it: small images the serial chain of their longest wave (steps,
-// fetches, accumulation), large ones vector issue and L1 lookups together
-// (isosurface 1024^2 over 4.4 M slab points: 315 M wave instructions, 0.51 ms
-// of the 0.52; 272 M cache-line lookups).  Hence, with the same arithmetic:
+// fetches, accumulation), large ones L1 lookups and vector issue together
+// (isosurface 1024^2 over 4.4 M slab points, 0.51 ms: 299 M cache-line lookups,
+// 0.49 ms at one a cycle and CU, 262 M vector instructions of a wave, 0.43 ms;
+// emission-absorption 512^2 of 2 M clustered points, 1.20 ms: 0.77 and 0.55).
+// Hence, with the same arithmetic:
 // the walk and the march are decoupled (ray_cast), so lanes do not wait for
 // each other at brick borders; a level's facts, the child list and the exit
 // time stay in registers and LDS instead of being re-read through per-lane
@@ -178,12 +180,12 @@ template <int L>
 struct RenderShared {
     LevelInfo lev[MAXLEV];
     uint2 queue[QUEUE][64 / L];     // leaf index, entry time
-    int nodeid[MAXLEV][64 / L];     // (the last two: only the tree's levels are allocated)
+    int nodeid[MAXLEV][64 / L];     // (all MAXLEV levels: 9.5 KB a workgroup for L = 1, 2.6 KB for L = 4)
     float tMax[MAXLEV][64 / L];
 };
 
 __device__ inline bool inside(f3 p, float r0) {
-    // (a NaN comes with infinities or NaNs on the other axes, which fail)
+    // (a NaN fails, or, alone on its axis, gives taps that are NaN and pass no test)
     return fminf(fminf(p.x, p.y), p.z) >= 0.0f && fmaxf(fmaxf(p.x, p.y), p.z) < r0;
 }
 
@@ -736,8 +738,10 @@ __device__ inline void k_render_body(const RenderArgs& A, uint32_t bid, RenderSh
 
 // One 64-thread workgroup per pixel tile; several grids' images in one launch.
 // Occupancy asked of the compiler: four waves per SIMD (128 VGPRs) hold the
-// taps of four samples; five spill there (isosurface 1024^2 0.52 -> 1.2 ms)
-// and three gain nothing.  One sample or two, or one per lane, fit five.
+// taps of four samples, but for 17 to 20 words of the isosurface's FP32 form;
+// five spill there (isosurface 1024^2 0.52 -> 1.2 ms) and three gain nothing.
+// One sample or two, or one per lane, are compiled for five (two samples spill 3
+// to 17 words); with one lane per ray the 9.5 KB of LDS allow 17 waves a CU.
 template <int MODE, typename AT, int U, int L, int BR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(U == 4 ? 4 : 5))) void k_render(RenderArgs a0,
                                                                                                     MultiMap m) {

@@ -321,7 +321,7 @@ private:
     int bkt_scs_ = 0, bkt_R_ = 0;
     float bkt_radius_ = 0.f;
     int bkt_n_ = 0;                // points of the insert
-    uint32_t bkt_fullest_ = ~0u;   // no subcell holds more points (~0: not known)
+    uint32_t bkt_fullest_ = ~0u;   // no subcell holds more points: the gather's dense line where none passes it, else ~0
     unsigned bkt_gen_ = ~0u;       // topology generation of the current buckets
 
     // topology scratch
