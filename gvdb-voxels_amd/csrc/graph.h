@@ -11,7 +11,7 @@
 //
 // A replay runs the recorded launches with their recorded arguments (point
 // count, radius, camera) over the current contents of the device buffers
-// (points, atlas, render buffers).  It is refused when the topology of a
+// (points, buckets, atlas, render buffers, the committed transfer function).  It is refused when the topology of a
 // grid changed or any library buffer was reallocated since the capture; the
 // insert's points must still fall inside the topology (a replay whose insert
 // met a point outside every brick reports GVDB_ERR_STATE at

@@ -2,7 +2,8 @@
 the oracle: blobs that fill bricks, fill part of them, or lie on a few voxels,
 near the origin too (where the distances are float), at the radii of every
 variant, FP32 and FP16, one grid, a batch and a graph replay; repeated gathers
-after one insert (the list of dense bricks is reused)."""
+after one insert (the list of dense bricks is reused); gathers recorded without
+their insert, after a replayed insert and after a refused recording."""
 import numpy as np
 import pytest
 
