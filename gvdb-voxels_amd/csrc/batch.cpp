@@ -74,6 +74,7 @@ int Batch::enter(Volume* const* v, int G, int* failed) {
                 }
                 return GVDB_ERR_STATE;
             }
+            cap_->note(v[g]);   // capture_end takes every noted grid out of the recording again
             v[g]->set_capture(cap_);
             continue;
         }

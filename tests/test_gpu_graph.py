@@ -165,6 +165,37 @@ def test_calls_outside_the_chain_fail_the_recording(gpu):
     v.close()
 
 
+def test_call_outside_the_chain_fails_a_batch_recording(gpu):
+    """A refused call in a batch's recording fails it and leaves no grid behind
+    in it: batched and single calls run directly afterwards."""
+    from gvdb_amd import workloads as Wk
+    c = (64.0, 64.0, 64.0)
+    sets = [Wk.sphere_shell(4000, seed=44 + k, radius=25.0 + k, centre=c) for k in range(3)]
+    vols = [_grid(gpu, p, c) for p in sets]
+    ns = [len(p) for p in sets]
+    B = gpu.GridBatch(0, 3)
+    lens = B.InsertPointsSubcell(vols, 4, ns, R)
+    B.GatherDensity(vols, 4, lens, R, 0)
+    B.synchronize()
+    B.CaptureBegin()
+    with pytest.raises(gpu.GVDBError):
+        B.RebuildTopology(vols, ns, R)
+    with pytest.raises(gpu.GVDBError):
+        B.CaptureEnd()
+    B.ClearChannel(vols, 0)
+    assert np.array_equal(B.InsertPointsSubcell(vols, 4, ns, R), lens)
+    B.synchronize()
+    B.close()
+    for v, n in zip(vols, ns):
+        v.RequestFullRebuild(True)
+        v.RebuildTopology(n, R, H.ZERO3)
+        v.FinishTopology(False, True)
+        v.UpdateAtlas()
+        _chain(gpu, v, n)
+        v.synchronize()
+        v.close()
+
+
 def test_graph_replay_batch(gpu):
     from gvdb_amd import workloads as Wk
     grids = [Wk.sphere_shell(4000 + 3000 * k, seed=50 + k, radius=20.0 + 8 * k, centre=(80.0 + 20 * k, 90.0, 100.0))
