@@ -919,7 +919,7 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
                 na.push_back(NbrArgs{pl.t, v->nbr_.as<int>(), int(pl.numMap), v->nmask_.as<uint32_t>(),
                                      v->nbase_.as<long long>(), v->brick_tab(), v->bkt_cnt_.as<uint32_t>(), pl.spb,
                                      v->lenparts_.as<u64>(), small(g, SM_ORPHANS)});
-                v->nbr_gen_ = v->topo_gen_;
+                if (!ex.cap) v->nbr_gen_ = v->topo_gen_;   // recorded, not run
             } else {
                 fa.push_back(FillArgs{v->bkt_cnt_.p, pl.numMap * u64(pl.spb), 0, 0});
                 fa.push_back(FillArgs{small(g, SM_ORPHANS), 1, 0, 0});
@@ -1287,7 +1287,7 @@ int Volume::multi_apron(Volume* const* vs, int G, int c, float boundval, const E
             XCHK(v, v->nbase_.ensure(size_t(bricks) * 27 * 8));
             na.push_back(NbrArgs{t, v->nbr_.as<int>(), bricks, v->nmask_.as<uint32_t>(), v->nbase_.as<long long>(),
                                  v->brick_tab()});
-            v->nbr_gen_ = v->topo_gen_;
+            if (!ex.cap) v->nbr_gen_ = v->topo_gen_;   // recorded, not run
         }
         const bool faces = v->faces_chan_ == c && v->faces_epoch_ == v->atlas_epoch_ && v->faces_topo_ == v->topo_gen_;
         aa.push_back(ApronArgs{t, v->nbase_.as<long long>(), v->nbr_.as<int>(),

@@ -165,6 +165,55 @@ def test_calls_outside_the_chain_fail_the_recording(gpu):
     v.close()
 
 
+def test_neighbour_table_of_a_recording_is_not_taken_as_built(gpu):
+    """The chain recorded first on a new topology: refused where buffers had to
+    grow, and not launched where they did not; the direct chain afterwards, and
+    an UpdateApron by itself, build the neighbour table themselves."""
+    from gvdb_amd import workloads as Wk
+    c = (96.0, 96.0, 96.0)
+    pts = Wk.sphere_shell(20000, seed=45, radius=40.0, centre=c)
+    other = Wk.sphere_shell(20000, seed=46, radius=38.0, centre=(88.0, 104.0, 96.0))
+
+    def direct(p):
+        w = _grid(gpu, p, c)
+        _chain(gpu, w, len(p))
+        w.synchronize()
+        s = _state(w)
+        w.close()
+        return s
+
+    want, want2 = direct(pts), direct(other)
+    v = _grid(gpu, pts, c)
+    v.Render(gpu.SHADE_VOLUME, 0, 0)     # commits the transfer function
+    v.synchronize()
+    v.CaptureBegin()
+    _chain(gpu, v, len(pts))
+    with pytest.raises(gpu.GVDBError) as e:
+        v.CaptureEnd()
+    assert e.value.code == gpu.ERR_STATE
+    _chain(gpu, v, len(pts))
+    v.synchronize()
+    assert all(np.array_equal(a, b) for a, b in zip(_state(v), want))
+    # a topology of fewer bricks in the buffers there are
+    v.SetPoints(other)
+    v.RequestFullRebuild(True)
+    v.RebuildTopology(len(other), R, H.ZERO3)
+    v.FinishTopology(False, True)
+    v.UpdateAtlas()
+    v.CaptureBegin()
+    _chain(gpu, v, len(other))
+    g = v.CaptureEnd()
+    _chain(gpu, v, len(other))
+    v.synchronize()
+    assert all(np.array_equal(a, b) for a, b in zip(_state(v), want2))
+    _wipe(gpu, v)
+    g.launch()
+    g.synchronize()
+    assert all(np.array_equal(a, b) for a, b in zip(_state(v), want2))
+    g.close()
+    v.close()
+
+
 def test_call_outside_the_chain_fails_a_batch_recording(gpu):
     """A refused call in a batch's recording fails it and leaves no grid behind
     in it: batched and single calls run directly afterwards."""
