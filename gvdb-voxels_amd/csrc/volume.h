@@ -176,7 +176,14 @@ public:
     // per-frame chain are recorded into it instead of run
     bool capturing() const { return capture_ != nullptr; }
     Graph* capture() const { return capture_; }
-    void set_capture(Graph* g) { capture_ = g; }
+    // into a recording (g) or out of it (null).  Boundary layers of a gather
+    // serve the aprons on their side only: a recorded apron the gather recorded
+    // before it, a direct one the direct gather with no replay since.
+    void set_capture(Graph* g) {
+        if (g != capture_) forget_faces();
+        capture_ = g;
+    }
+    void forget_faces() { faces_epoch_ = ~0u; }
     // fails the recording with `code` (a call that cannot be recorded)
     int not_recordable(const char* what);
     std::shared_ptr<SharedStream> stream_owner() const { return cur_stream_; }

@@ -214,6 +214,78 @@ def test_neighbour_table_of_a_recording_is_not_taken_as_built(gpu):
     v.close()
 
 
+def _padded(v):
+    return v.atlas().view(np.uint32).copy()
+
+
+def test_aprons_and_recordings_use_their_own_boundary_layers(gpu):
+    """UpdateApron after GatherDensity reads the layers the gather left; not
+    those of a gather that is only recorded, nor from before a replay that wrote
+    the atlas, nor, recorded alone, those current at the recording.  Each is
+    compared with an UpdateApron that reads the bricks (after an operator that
+    changes nothing: noise of amplitude 0)."""
+    from gvdb_amd import workloads as Wk
+    c = (96.0, 96.0, 96.0)
+    pts = Wk.sphere_shell(20000, seed=47, radius=40.0, centre=c)
+    n = len(pts)
+    v = _grid(gpu, pts, c)
+    ln = _chain(gpu, v, n)
+    v.synchronize()
+
+    def apron_from_bricks():
+        v.Compute(gpu.FUNC_NOISE, 0, 1, (0.0, 0.0, 0.0), False, True, 0.0)
+        v.UpdateApron(0, 0.0)
+        v.synchronize()
+        return _padded(v)
+
+    def shrink():
+        # interiors and aprons no longer the gather's
+        v.Compute(gpu.FUNC_SMOOTH, 0, 1, (1.0, 0.0, 0.0), False, True, 0.0)
+
+    # a gather and an apron recorded, not launched; then a direct apron
+    shrink()
+    v.CaptureBegin()
+    v.GatherDensity(4, n, R, H.ZERO3, ln, 0, 0, False)
+    v.UpdateApron(0, 0.0)
+    both = v.CaptureEnd()
+    v.UpdateApron(0, 0.0)
+    v.synchronize()
+    a = _padded(v)
+    assert np.array_equal(a, apron_from_bricks())
+    # an apron recorded alone right after a direct gather, replayed over other voxels
+    v.GatherDensity(4, n, R, H.ZERO3, ln, 0, 0, False)
+    v.CaptureBegin()
+    v.UpdateApron(0, 0.0)
+    alone = v.CaptureEnd()
+    for _ in range(2):
+        shrink()
+        alone.launch()
+        alone.synchronize()
+        a = _padded(v)
+        assert np.array_equal(a, apron_from_bricks())
+    # the channel cleared by a replay between a direct gather and its apron
+    v.CaptureBegin()
+    v.ClearChannel(0)
+    clear = v.CaptureEnd()
+    v.GatherDensity(4, n, R, H.ZERO3, ln, 0, 0, False)
+    clear.launch()
+    clear.synchronize()
+    v.UpdateApron(0, 0.0)
+    v.synchronize()
+    assert not _padded(v).any()
+    # the recorded pair against the direct one
+    both.launch()
+    both.synchronize()
+    a = _padded(v)
+    v.GatherDensity(4, n, R, H.ZERO3, ln, 0, 0, False)
+    v.UpdateApron(0, 0.0)
+    v.synchronize()
+    assert a.any() and np.array_equal(a, _padded(v)) and np.array_equal(a, apron_from_bricks())
+    for g in (both, alone, clear):
+        g.close()
+    v.close()
+
+
 def test_call_outside_the_chain_fails_a_batch_recording(gpu):
     """A refused call in a batch's recording fails it and leaves no grid behind
     in it: batched and single calls run directly afterwards."""
