@@ -127,13 +127,14 @@ int graph_launch(Graph* g, std::string& err) {
             return GVDB_ERR_STATE;
         }
     (void)hipSetDevice(g->device);
-    for (Volume* v : g->vols) v->forget_faces();   // the replay may write the atlas
-    for (const Graph::Insert& in : g->inserts) in.v->forget_fullest();   // a gather may come before graph_synchronize
     hipError_t e = hipGraphLaunch(g->exec, g->stream);
     if (e != hipSuccess) {
         err = std::string("graph launch: ") + hipGetErrorString(e);
         return GVDB_ERR_HIP;
     }
+    // direct calls may come before graph_synchronize
+    for (Volume* v : g->vols) v->forget_faces();   // the replay may write the atlas
+    for (const Graph::Insert& in : g->inserts) in.v->set_insert_state(in.state);
     g->pending = true;
     return GVDB_OK;
 }

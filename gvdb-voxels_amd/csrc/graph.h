@@ -9,6 +9,9 @@
 // subcell entry count) stays on the device and reaches pinned host memory
 // through a copy recorded in the graph, read by graph_synchronize.
 //
+// Recorded calls see what was recorded before them, direct calls what ran:
+// a direct gather uses the recorded insert's buckets from the replay on.
+//
 // A replay runs the recorded launches with their recorded arguments (point
 // count, radius, camera) over the current contents of the device buffers
 // (points, buckets, atlas, render buffers, the committed transfer function).  It is refused when the topology of a
@@ -42,6 +45,7 @@ struct Graph {
     struct Insert {
         Volume* v;
         const uint32_t* slot;             // pinned words the recorded readback fills
+        Volume::InsertState state;        // what it leaves, once a replay has run it
     };
     std::vector<Insert> inserts;
     unsigned long long alloc_gen = 0;

@@ -1004,7 +1004,7 @@ int Volume::multi_insert(Volume* const* vs, int G, int scs, const int* n, const 
             v->bkt_n_ = n[g];
             v->bkt_gen_ = v->topo_gen_;
             v->forget_fullest();
-            ex.cap->inserts.push_back(Graph::Insert{v, ex.hsmall + size_t(g) * SMALL_WORDS});
+            ex.cap->inserts.push_back(Graph::Insert{v, ex.hsmall + size_t(g) * SMALL_WORDS, v->insert_state()});
         }
         return GVDB_OK;
     }

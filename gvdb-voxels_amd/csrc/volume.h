@@ -179,11 +179,35 @@ public:
     // into a recording (g) or out of it (null).  Boundary layers of a gather
     // serve the aprons on their side only: a recorded apron the gather recorded
     // before it, a direct one the direct gather with no replay since.
+    // What the last insert left belongs to its side too: the recorded calls see
+    // the recorded insert, the direct ones theirs again afterwards, and the
+    // recorded one's once a replay has run it.
     void set_capture(Graph* g) {
-        if (g != capture_) forget_faces();
+        if (g == capture_) return;
+        forget_faces();
+        if (!capture_) direct_insert_ = insert_state();
+        if (!g) set_insert_state(direct_insert_);
         capture_ = g;
     }
     void forget_faces() { faces_epoch_ = ~0u; }
+    struct InsertState {
+        int num_sc, map_n, scs, R, n;
+        float radius;
+        uint32_t fullest;
+        unsigned sc_gen, bkt_gen;
+        bool pull, stale, map_ready, sc16, clr;
+    };
+    InsertState insert_state() const {
+        return InsertState{num_sc_, sc_map_n_, bkt_scs_, bkt_R_, bkt_n_, bkt_radius_, bkt_fullest_, sc_gen_, bkt_gen_,
+                           last_insert_pull_, entries_stale_, map_ready_, sc16_valid_, bkt_clr_};
+    }
+    void set_insert_state(const InsertState& s) {
+        num_sc_ = s.num_sc; sc_map_n_ = s.map_n; bkt_scs_ = s.scs; bkt_R_ = s.R; bkt_n_ = s.n;
+        bkt_radius_ = s.radius;
+        bkt_fullest_ = s.fullest;
+        sc_gen_ = s.sc_gen; bkt_gen_ = s.bkt_gen;
+        last_insert_pull_ = s.pull; entries_stale_ = s.stale; map_ready_ = s.map_ready; sc16_valid_ = s.sc16; bkt_clr_ = s.clr;
+    }
     // fails the recording with `code` (a call that cannot be recorded)
     int not_recordable(const char* what);
     std::shared_ptr<SharedStream> stream_owner() const { return cur_stream_; }
@@ -303,6 +327,7 @@ private:
     unsigned nbr_gen_ = ~0u;
     void* noalloc_ = nullptr;   // this device's copy of the no-allocation scratch array
     Graph* capture_ = nullptr;      // the graph being recorded, if any
+    InsertState direct_insert_{};   // while recording: what the last direct insert left
     std::vector<Graph*> graphs_;    // graphs that replay calls on this grid
 
     // points

@@ -286,6 +286,58 @@ def test_aprons_and_recordings_use_their_own_boundary_layers(gpu):
     v.close()
 
 
+def test_a_recorded_insert_counts_from_its_replay_on(gpu):
+    """What an insert leaves for gathers and reads: the direct one's until a
+    replay runs the recorded one (another radius here), with its own entry
+    tables after every replay; none after a refused recording."""
+    from gvdb_amd import workloads as Wk
+    c = (96.0, 96.0, 96.0)
+    pts = Wk.sphere_shell(20000, seed=48, radius=40.0, centre=c)
+    sets = [pts, (c + (pts - c) * np.float32(0.98)).astype(np.float32)]
+    n = len(pts)
+    v = _grid(gpu, pts, c)
+    v.CaptureBegin()
+    v.InsertPointsSubcell(4, n, R, H.ZERO3)
+    with pytest.raises(gpu.GVDBError):      # buffers had to grow
+        v.CaptureEnd()
+    with pytest.raises(gpu.GVDBError) as e:
+        v.GatherLevelSet(4, n, R, H.ZERO3, 0, 0, 0, False)
+    assert e.value.code == gpu.ERR_STATE
+
+    def gather(p, r, ln=None):
+        if ln is None:
+            v.SetPoints(p)
+            ln = v.InsertPointsSubcell(4, n, r, H.ZERO3)
+        v.ClearChannel(0)
+        v.GatherDensity(4, n, r, H.ZERO3, ln, 0, 0, False)
+        v.UpdateApron(0, 0.0)
+        v.synchronize()
+        return _padded(v), ln
+
+    want = {}
+    for k, p in enumerate(sets):
+        want[k], ln = gather(p, 1.0)
+        want[k] = (want[k], ln, v.subcells())
+    want2, ln2 = gather(pts, R)
+    assert not np.array_equal(want[0][0], want[1][0]) and not np.array_equal(want[0][0], want2)
+    v.CaptureBegin()
+    v.InsertPointsSubcell(4, n, 1.0, H.ZERO3)
+    g = v.CaptureEnd()
+    assert np.array_equal(gather(None, R, ln2)[0], want2)      # not launched yet
+    for k in (1, 0, 1):
+        v.SetPoints(sets[k])
+        g.launch()
+        g.synchronize()
+        a, ln, tables = want[k]
+        assert np.array_equal(gather(None, 1.0, ln)[0], a)
+        t = v.subcells()
+        assert all(np.array_equal(t[x], tables[x]) for x in ("cnt", "off", "pos", "nid"))
+        b, l2 = gather(pts, R)                                  # a direct insert takes over
+        assert l2 == ln2 and np.array_equal(b, want2)
+    g.close()
+    v.close()
+
+
 def test_call_outside_the_chain_fails_a_batch_recording(gpu):
     """A refused call in a batch's recording fails it and leaves no grid behind
     in it: batched and single calls run directly afterwards."""
